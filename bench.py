@@ -109,10 +109,10 @@ def walk_drops(T, post, dev, S, C, N, K, rb):
     from torchtree_amd.likelihood import get_plan
 
     plan = get_plan(T, post, dev.index or 0)
-    d0, d1 = ctypes.c_int(), ctypes.c_int()
-    _lib.check(_lib.load().hx_plan_walk_info(plan.handle, None, None, None, ctypes.byref(d0),
-                                             ctypes.byref(d1)))
-    return d0.value
+    cherries = ctypes.c_int()
+    _lib.check(_lib.load().hx_plan_walk_info(plan.handle, None, None, ctypes.byref(cherries), None,
+                                             None))
+    return cherries.value if T > 2 else 0  # of two taxa the one cherry is the root
 
 
 def algorithmic_bytes(T, N, C, K, S, rb, nchunks, drops=0):
@@ -123,7 +123,7 @@ def algorithmic_bytes(T, N, C, K, S, rb, nchunks, drops=0):
     it does not store, and reads none back from HBM (a child that waited on the
     stack is re-read from L2), plus the tip codes. The four-state FP32 pre-order
     walk reads the same partials once (the adjoints live in registers), reads
-    each tip's 16-bit code once per sample and each dropped cherry's code pair,
+    each tip's code once per sample and each dropped cherry's two codes again,
     and writes the per-chunk branch statistics, which the reduction reads
     back. Otherwise the pre-order runs per level: each internal non-root node's
     L and its parent's U are read and its U written (3 P per node). Other state
@@ -141,7 +141,7 @@ def algorithmic_bytes(T, N, C, K, S, rb, nchunks, drops=0):
     else:
         post_b = 2 * (I - 1) * part + 2 * (I - 1) * K * N * 4 + tips + mats + weights
     if pre_walk_used(S, C, rb, N, K):
-        pre_b = (I - 1 - drops) * part + K * (T + drops) * N * 2 + mats + weights + 2 * gpart
+        pre_b = (I - 1 - drops) * part + K * (T + 2 * drops) * N + mats + weights + 2 * gpart
     else:
         pre_b = 3 * (I - 1) * part + tips + mats + weights + gpart
     return post_b, pre_b

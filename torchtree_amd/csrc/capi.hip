@@ -104,10 +104,13 @@ int hx_plan_create(int taxa, const int32_t* postorder, int device, hx_plan_t* ou
   }
   std::vector<int32_t> cher, cher_row;
   hx::list_cherries(T, kids, postorder, cher, cher_row);
-  std::vector<int32_t> prew;
-  int prew_depth = 0;
-  if (!hx::build_pre_walk(T, kids, postorder, prew, prew_depth, &drop, &cher_row)) {
-    hx::set_error("pre-order walk program construction failed");
+  std::vector<int32_t> prew, post4, pre4;
+  std::vector<uint8_t> drop4;
+  int prew_depth = 0, post4_slots = 0;
+  if (!hx::build_post4(T, walk, post4, post4_slots, drop4) ||
+      !hx::build_pre_walk(T, kids, postorder, prew, prew_depth, &drop4, &cher_row) ||
+      !hx::build_pre4(T, prew, drop4, pre4)) {
+    hx::set_error("walk program construction failed");
     return HX_ERR_BAD_TOPOLOGY;
   }
   auto* plan = new hx_plan_s();
@@ -118,14 +121,12 @@ int hx_plan_create(int taxa, const int32_t* postorder, int device, hx_plan_t* ou
   plan->root = root;
   plan->kids = kids;
   const size_t walk_off = hx::align_up(2 * (size_t)nn + 2 * (size_t)I, 4);
-  const size_t seg_off = walk_off + walk.size();
-  const size_t prew_off = hx::align_up(seg_off + segtab.size(), 4);
-  const size_t cher_off = prew_off + prew.size();
-  std::vector<int32_t> host(cher_off + cher.size(), 0);
+  const size_t post4_off = walk_off + walk.size();
+  const size_t pre4_off = post4_off + post4.size();
+  std::vector<int32_t> host(pre4_off + pre4.size(), 0);
   std::copy(walk.begin(), walk.end(), host.begin() + walk_off);
-  std::copy(segtab.begin(), segtab.end(), host.begin() + seg_off);
-  std::copy(prew.begin(), prew.end(), host.begin() + prew_off);
-  std::copy(cher.begin(), cher.end(), host.begin() + cher_off);
+  std::copy(post4.begin(), post4.end(), host.begin() + post4_off);
+  std::copy(pre4.begin(), pre4.end(), host.begin() + pre4_off);
   std::copy(kids.begin(), kids.end(), host.begin());
   int pos = 2 * nn;
   plan->post_off.push_back(0);
@@ -155,11 +156,10 @@ int hx_plan_create(int taxa, const int32_t* postorder, int device, hx_plan_t* ou
   plan->d_post = plan->d_buf + 2 * nn;
   plan->d_pre = plan->d_buf + 2 * nn + I;
   plan->d_walk = plan->d_buf + walk_off;
-  plan->d_segtab = plan->d_buf + seg_off;
-  plan->nseg = (int)(segtab.size() / hx::kWalkSegTips);
-  plan->d_prew = plan->d_buf + prew_off;
   plan->prew_depth = prew_depth;
-  plan->d_cher = plan->d_buf + cher_off;
+  plan->d_post4 = plan->d_buf + post4_off;
+  plan->d_pre4 = plan->d_buf + pre4_off;
+  plan->post4_slots = post4_slots;
   plan->ncher = (int)(cher.size() / 2);
   for (uint8_t b : drop) {
     plan->ndrop[0] += b & 1;

@@ -44,27 +44,25 @@ struct hx_plan_s {
   int I = 0;
   int root = 0;
   int32_t* d_buf = nullptr;   // device: kids[2(2T-1)] | post_nodes[I] | pre_nodes[I] | pad |
-                              //         walk[I][8] (16-byte aligned) | segtab[nseg][16] |
-                              //         prew[I][16] | cher[ncher][2]
+                              //         walk[I][8] (16-byte aligned) | post4[I][4] |
+                              //         pre4[I][16]
   const int32_t* d_kids = nullptr;
   const int32_t* d_post = nullptr;
   const int32_t* d_pre = nullptr;
   std::vector<int> post_off;  // host: level offsets into d_post (size levels+1)
   std::vector<int> pre_off;   // host: depth offsets into d_pre
   std::vector<int32_t> kids;  // host copy of kids
-  // Post-order walk program (walk.hpp): kWalkInts ints per internal node and
-  // the tip-segment table; the walk needs `walk_need` stack entries.
+  // Post-order walk program (walk.hpp): kWalkInts ints per internal node; the walk needs
+  // `walk_need` stack entries.
   const int32_t* d_walk = nullptr;
-  const int32_t* d_segtab = nullptr;
-  int nseg = 0;
   int walk_need = 0;
-  // Pre-order walk program (walk.hpp, build_pre_walk): kPreInts ints per
-  // internal node; its stack reaches `prew_depth` entries.
-  const int32_t* d_prew = nullptr;
-  int prew_depth = 0;
-  // Cherries (walk.hpp, list_cherries): [ncher][2] tip ids; how many the post-order walk
-  // drops under register mode 0 and 1.
-  const int32_t* d_cher = nullptr;
+  int prew_depth = 0;  // stack depth of the pre-order walk (walk.hpp, build_pre_walk)
+  // Programs of the four-state FP32 walks (walk.hpp, build_post4 and build_pre4) and the
+  // post-order one's exponent stack.
+  const int32_t* d_post4 = nullptr;
+  const int32_t* d_pre4 = nullptr;
+  int post4_slots = 0;
+  // Cherries, and how many build_walk's drop bits name under register mode 0 and 1.
   int ncher = 0;
   int ndrop[2] = {0, 0};
 };

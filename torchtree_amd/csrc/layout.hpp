@@ -67,12 +67,11 @@ inline int wide_nt(int C, int S, int rb) {
 // identical alone and in a batch.
 constexpr int kTargetChunks = 128;
 
-// The four-state FP32 pre-order walk with at most kPreWalkMaxC categories
+// The four-state FP32 passes with at most kPreWalkMaxC categories are walks
+// (pruning_walk.hip) at every size: choosing by size would make a sample's
+// FP32 gradient depend on the batch it is evaluated in. The pre-order walk
 // sums its branch statistics over the kPreWalkW tiles of a workgroup: one
-// chunk per kPreWalkW tiles. It serves every such call, also those with too
-// few workgroups (ceil(tiles / 4) x K) to fill the chip, where a pre-order by
-// level would be faster: choosing by size would make a sample's FP32 gradient
-// depend on the batch it is evaluated in.
+// chunk per kPreWalkW tiles.
 constexpr int kPreWalkW = 4;
 constexpr int kPreWalkMaxC = 4;
 inline bool use_pre_walk(int S, int C, int rb, int N, int K) {
@@ -145,8 +144,9 @@ inline WsLayout ws_layout_t(int taxa, int S, int N, int C, int K, int dtype, int
   if (grad_mode == 2) off = align_up(off + B * K * (size_t)t.nchunks * C * 8, 256);
   w.ppad = off;
   if (use_ppad(S, dtype, grad_mode)) off = align_up(off + B * K * (size_t)C * 2 * 64 * 64 * rb, 256);
-  // four-state FP32: 16-bit tip codes and cherry code pairs for the pre-order walk (a tree
-  // has at most T / 2 cherries)
+  // four-state FP32: room for 16-bit tip codes and cherry code pairs, which the walks no longer
+  // need (they read the caller's codes); kept so that workspace sizes, and the pattern slices
+  // chosen by them, stay as they are
   w.pcodes = off;
   if (S == 4 && rb == 4)
     off = align_up(off + ((size_t)taxa + (size_t)taxa / 2) * t.ntiles * 64 * 2, 256);
@@ -159,11 +159,9 @@ inline size_t workspace_bytes_for(int taxa, int S, int N, int C, int K, int dtyp
   return ws_layout_t(taxa, S, N, C, K, dtype, grad_mode).total;
 }
 
-// Register mode of the post-order walk's drop bits (walk.hpp) for a call, or -1 when every
-// internal partial is stored: cherries are dropped for four-state FP32 calls with tip codes
-// whose gradient runs as the pre-order walk (use_pre_walk), the only reader that rebuilds
-// them. Mode 0: the post-order walk keeps no stack depths in registers (mode 1 is the
-// program's mode for a walk that keeps depths 2..4 there).
+// Whether a call's walks leave cherries out of memory: 0 (the post-order walk stores no partial
+// of a cherry, the pre-order walk rebuilds it from the two tips' codes) for four-state FP32 calls
+// with tip codes that run as walks (use_pre_walk), -1 when every internal partial is stored.
 inline int walk_drop_mode(int S, int C, int N, int K, int dtype, int tip_kind) {
   if (S != 4 || dtype == HX_F64 || tip_kind != HX_TIPS_CODES || !use_pre_walk(S, C, 4, N, K))
     return -1;

@@ -222,6 +222,14 @@ static int validate(const CallArgs& c) {
   return HX_OK;
 }
 
+// Whether a call's two passes run as the FP32 walks of pruning_walk.hip: their tip codes are one
+// buffer of 32-bit offsets, so alignments of 4 GiB of codes and more take the other four-state
+// kernels, which store every cherry.
+static bool runs_walk4(const CallArgs& c) {
+  return c.dtype != HX_F64 && use_pre_walk(c.S, c.C, 4, c.N, c.K) &&
+         (c.tip_kind != HX_TIPS_CODES || (size_t)c.plan->T * c.N < ((size_t)1 << 32));
+}
+
 template <typename R>
 static PassArgs<R> make_args(const CallArgs& c) {
   const WsLayout w = ws_layout(c.plan, c.S, c.N, c.C, c.K, c.dtype, c.grad_mode);
@@ -257,10 +265,7 @@ static PassArgs<R> make_args(const CallArgs& c) {
   a.gtau = reinterpret_cast<double*>(base + w.gpart);
   a.ppad = use_ppad(c.S, c.dtype, c.grad_mode) ? reinterpret_cast<R*>(base + w.ppad) : nullptr;
   a.split = c.dtype == HX_F32_BF16X3;
-  a.drop_mode = walk_drop_mode(c.S, c.C, c.N, c.K, c.dtype, c.tip_kind);
-  a.cher = c.plan->d_cher;
-  a.ncher = c.plan->ncher;
-  a.pcodes = c.S == 4 && sizeof(R) == 4 ? reinterpret_cast<uint16_t*>(base + w.pcodes) : nullptr;
+  a.drop = runs_walk4(c) && walk_drop_mode(c.S, c.C, c.N, c.K, c.dtype, c.tip_kind) >= 0;
   return a;
 }
 
@@ -270,8 +275,21 @@ static int run_post(const CallArgs& c, double* out_l, double* out_f, double* out
   const hx_plan_s* plan = c.plan;
   int nparts = a.nchunks;
   if (c.S == 4) {
-    const int rc = launch_post_dna<R>(a, plan->d_walk, plan->d_segtab, plan->nseg, plan->I,
-                                      plan->walk_need, c.tip_kind, st);
+    int rc = HX_OK;
+    if constexpr (std::is_same<R, float>::value) {
+      if (runs_walk4(c)) {
+        HX_REQUIRE(dna_walk_lds(plan->T, 1, plan->walk_need, c.tip_kind, c.ncodes, 4) <= kDnaWalkLdsMax,
+                   HX_ERR_UNSUPPORTED, "post-order walk: too many taxa");
+        // no gradient can follow in a workspace that has no room for one (each gradient call
+        // checks for its own): then the partials need not be kept
+        const bool store = c.ws_bytes >= ws_layout(plan, c.S, c.N, c.C, c.K, c.dtype, 2).total;
+        rc = launch_post_walk4(a, plan->d_post4, plan->I, plan->post4_slots, c.tip_kind, store, st);
+      } else {
+        rc = launch_post_dna<R>(a, plan->d_walk, plan->I, plan->walk_need, c.tip_kind, st);
+      }
+    } else {
+      rc = launch_post_dna<R>(a, plan->d_walk, plan->I, plan->walk_need, c.tip_kind, st);
+    }
     if (rc != HX_OK) return rc;
     nparts = a.ntiles;
   } else {
@@ -308,12 +326,12 @@ static int run_pre(const CallArgs& c, double* out, hipStream_t st) {
     HX_HIP_TRY(hipGetLastError());
   }
   if constexpr (std::is_same<R, float>::value) {
-    if (use_pre_walk(c.S, c.C, 4, c.N, c.K)) {
-      const int rc = launch_pre_walk(a, plan->d_prew, plan->I, c.tip_kind, st);
+    if (runs_walk4(c)) {
+      const int rc = launch_pre_walk4(a, plan->d_pre4, plan->I, c.tip_kind, st);
       if (rc != HX_OK) return rc;
     }
   }
-  for (int d = 0; d < D && !(sizeof(R) == 4 && use_pre_walk(c.S, c.C, 4, c.N, c.K)); ++d) {
+  for (int d = 0; d < D && !runs_walk4(c); ++d) {
     const int off = plan->pre_off[d], width = plan->pre_off[d + 1] - off;
     const int rc = c.S == 4
                        ? launch_pre_dna<R>(a, plan->d_pre + off, width, c.tip_kind, d == 0, st)

@@ -31,13 +31,9 @@ struct PassArgs {
   R* ppad;                // [K][B][C][2][64][64]: P and P^T zero-padded (FP32, 33..64 states);
                           // with `split`, each element holds its BF16 hi and lo halves
   int split;              // dense-state products as split BF16 on the matrix cores (FP32 only)
-  // Four-state FP32 walks with tip codes: -1, or the register mode whose drop bits
-  // (walk.hpp) apply: the post-order walk stores no partial of those cherries and the
-  // pre-order walk rebuilds it from pcodes.
-  int drop_mode;
-  const int32_t* cher;    // [ncher][2] tip ids of the cherries
-  int ncher;
-  uint16_t* pcodes;       // [T + ncher][np]: tip codes, then each cherry's two codes (lo | hi << 8)
+  // Four-state FP32 walks with tip codes: the post-order stores no cherry's partial and the
+  // pre-order rebuilds it from the two tips' codes.
+  int drop;
 };
 
 constexpr double kLn2 = 0.69314718055994530942;
@@ -60,20 +56,29 @@ template <typename R>
 int launch_pre_wide(const PassArgs<R>& a, const int32_t* nodes, int width, int tips, bool root,
                     int S, hipStream_t st);
 
-// Four-state kernels (pruning_dna.hip): fused post-order walk and the
-// pre-order adjoint one level per launch. Partials of S = 4 use the
-// category-major layout [slot][K][C][np][4].
+// Four-state kernels. Partials of S = 4 use the category-major layout [slot][K][C][np][4].
+// FP32 at up to kPreWalkMaxC categories: both passes as walks on the matrix cores
+// (pruning_walk.hip; use_pre_walk in layout.hpp). `store`: keep the partials for a gradient.
+int launch_post_walk4(const PassArgs<float>& a, const int32_t* prog, int nprog, int slots, int tips,
+                      bool store, hipStream_t st);
+int launch_pre_walk4(const PassArgs<float>& a, const int32_t* prog, int nprog, int tips,
+                     hipStream_t st);
+// FP64, and FP32 at more categories (pruning_dna.hip): the post-order walk on the vector units
+// and the pre-order adjoint one level per launch.
 constexpr size_t kDnaLdsBudget = 64 * 1024;
 constexpr size_t kDnaWalkLdsMax = 160 * 1024;  // gfx950 LDS per workgroup
+// LDS of that post-order walk with W samples per block: it bounds the taxa of every four-state call
+// with tip codes (about 2,500).
+inline size_t dna_walk_lds(int T, int W, int need, int tips, int ncodes, size_t rb) {
+  return (tips == HX_TIPS_CODES ? (size_t)T * 64 + (size_t)ncodes * 4 * rb : 0) +
+         (size_t)W * need * 64 * 4;
+}
 template <typename R>
-int launch_post_dna(const PassArgs<R>& a, const int32_t* prog, const int32_t* segtab, int nseg,
-                    int nprog, int need, int tips, hipStream_t st);
+int launch_post_dna(const PassArgs<R>& a, const int32_t* prog, int nprog, int need, int tips,
+                    hipStream_t st);
 template <typename R>
 int launch_pre_dna(const PassArgs<R>& a, const int32_t* nodes, int width, int tips, bool root,
                    hipStream_t st);
-// The whole pre-order in one launch (FP32, C <= kPreWalkMaxC; use_pre_walk).
-int launch_pre_walk(const PassArgs<float>& a, const int32_t* prog, int nprog, int tips,
-                    hipStream_t st);
 
 // Dense-state kernels on MFMA (pruning_mfma.hip, FP32 and FP64); used when
 // use_mfma() (layout.hpp).

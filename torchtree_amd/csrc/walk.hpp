@@ -251,4 +251,131 @@ inline bool build_pre_walk(int T, const std::vector<int32_t>& kids, const int32_
   return (int)prog.size() == kPreInts * I && prog[0] == root && pend.empty() && depth <= 255;
 }
 
+// ------------------------------------------------- programs of the FP32 walks
+// The matrix-core walks of the four-state FP32 passes (pruning_walk.hip) run the same node
+// orders from more compact programs, derived from build_walk and build_pre_walk.
+//
+// Post-order, kPost4Ints ints per internal node in walk order, the children ordered so that
+// child 2 is the previous entry's result whenever there is one:
+//   [0] child 1  [1] child 2  [2] node
+//   [3] bits 0-1 type: 0 both tips; 1 a tip and the previous result; 2 the held result and
+//                the previous one; 3 a spilled result and the previous one
+//       bit 2 hold: the previous result waits in registers from before this entry
+//       bit 3 drop: a cherry that no walk reads from memory (its partial is not stored)
+//       bit 4 spill: the node's result waits in memory, its exponent in stack slot [16-23]
+//       bits 8-15 the slot of the spilled child (type 3)
+// A join's first-evaluated child is held in registers when the other child's subtree needs
+// no waiting result itself (a caterpillar), so one held result suffices; otherwise it is
+// spilled: read back from its stored partial.
+constexpr int kPost4Ints = 4;
+
+inline bool build_post4(int T, const std::vector<int32_t>& walk, std::vector<int32_t>& prog,
+                        int& slots, std::vector<uint8_t>& drop) {
+  const int I = T - 1, nn = 2 * T - 1;
+  std::vector<int> at(nn, -1);
+  std::vector<int> type(I), flags(I, 0), first(I, -1);
+  for (int i = 0; i < I; ++i) at[walk[(size_t)kWalkInts * i]] = i;
+  std::vector<char> waits(nn, 0);  // spilled nodes
+  int last_join = -1;              // latest entry with a waiting child
+  for (int i = 0; i < I; ++i) {
+    const int32_t* e = walk.data() + (size_t)kWalkInts * i;
+    const int kl = e[6] & 0xff, kr = (e[6] >> 8) & 0xff;
+    if (kl == 2 || kr == 2) {
+      first[i] = kl == 2 ? e[1] : e[2];
+      const int start = at[first[i]] + 1;  // the other child's first entry
+      if (start <= 0 || start >= i) return false;
+      if (last_join < start) {
+        type[i] = 2;
+        flags[start] |= 1 << 2;
+      } else {
+        type[i] = 3;
+        waits[first[i]] = 1;
+      }
+      last_join = i;
+    } else {
+      type[i] = (kl == 0 && kr == 0) ? 0 : 1;
+    }
+  }
+  drop.assign(nn, 0);
+  prog.clear();
+  prog.reserve((size_t)kPost4Ints * I);
+  std::vector<int> stack;
+  slots = 0;
+  for (int i = 0; i < I; ++i) {
+    const int32_t* e = walk.data() + (size_t)kWalkInts * i;
+    const int v = e[0], a = e[1], b = e[2], kr = (e[6] >> 8) & 0xff;
+    // child 2: the previous result, or the right tip of a cherry
+    const bool swap = type[i] != 0 && kr != 1;
+    int m = type[i] | flags[i];
+    if (type[i] == 3) {
+      if (stack.empty() || stack.back() != first[i]) return false;
+      stack.pop_back();
+      m |= (int)stack.size() << 8;
+    }
+    if (waits[v]) {
+      m |= (1 << 4) | ((int)stack.size() << 16);
+      stack.push_back(v);
+      slots = std::max(slots, (int)stack.size());
+    } else if (a < T && b < T && i + 1 < I) {
+      m |= 1 << 3;
+      drop[v] = 1;
+    }
+    const int32_t w[kPost4Ints] = {swap ? b : a, swap ? a : b, v, m};
+    prog.insert(prog.end(), w, w + kPost4Ints);
+  }
+  return stack.empty() && slots <= 255;
+}
+
+// Pre-order, kPre4Ints ints per internal node in the order of build_pre_walk, the children
+// ordered so that child 2 is the one the walk continues into and child 1 the pushed one:
+//   [0] node  [1] child 1  [2] child 2
+//   [3] bits 0-1 the node's adjoint: 0 root, 1 the continuation, 2 a pop from memory, 3 the
+//                held one
+//       bits 2-3, 4-5 child 1's, child 2's partial: 0 tip, 1 dropped (a cherry rebuilt from
+//                its two tips), 2 stored
+//       bits 6-7 child 1's adjoint: 0 none, 1 pushed to its partial's place, 2 held
+//       bit 8 the walk continues into child 2
+//   [4], [5] a dropped child 1's two tips, [6], [7] those of child 2 (otherwise 0)
+//   [8] .. [15] 0
+// An adjoint is held in registers when nothing else is pushed until its pop, which leaves at
+// most one held adjoint.
+constexpr int kPre4Ints = 16;
+
+inline bool build_pre4(int T, const std::vector<int32_t>& pre, const std::vector<uint8_t>& drop,
+                       std::vector<int32_t>& prog) {
+  const int I = T - 1;
+  std::vector<int> push_at, held(I, 0), from_hold(I, 0);
+  int last_push = -1;
+  for (int i = 0; i < I; ++i) {
+    const int32_t* e = pre.data() + (size_t)kPreInts * i;
+    if ((e[3] & 3) == 2) {
+      if (push_at.empty()) return false;
+      const int j = push_at.back();
+      push_at.pop_back();
+      held[j] = from_hold[i] = last_push == j;
+    }
+    if (e[5] >= 0) {
+      push_at.push_back(i);
+      last_push = i;
+    }
+  }
+  prog.clear();
+  prog.reserve((size_t)kPre4Ints * I);
+  for (int i = 0; i < I; ++i) {
+    const int32_t* e = pre.data() + (size_t)kPreInts * i;
+    const bool swap = e[4] == 0;  // the walk continues into a
+    const int c1 = e[swap ? 2 : 1], c2 = e[swap ? 1 : 2];
+    auto kind = [&](int ch) { return ch < T ? 0 : (drop[ch] ? 1 : 2); };
+    const int src = (e[3] & 3) == 2 ? (from_hold[i] ? 3 : 2) : (e[3] & 3);
+    const int push = e[5] < 0 ? 0 : (held[i] ? 2 : 1);
+    const int m = src | (kind(c1) << 2) | (kind(c2) << 4) | (push << 6) | (e[4] >= 0 ? 1 << 8 : 0);
+    const int32_t* g1 = e + (swap ? 12 : 10);
+    const int32_t* g2 = e + (swap ? 10 : 12);
+    const int32_t w[kPre4Ints] = {e[0],  c1,    c2, m, g1[0], g1[1], g2[0], g2[1],
+                                  0, 0, 0, 0, 0, 0, 0, 0};
+    prog.insert(prog.end(), w, w + kPre4Ints);
+  }
+  return push_at.empty();
+}
+
 }  // namespace hx

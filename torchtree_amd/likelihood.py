@@ -242,8 +242,9 @@ class Pruning:
 
     def _launches(self, which, S, C, code, K):
         """Kernel launches of one pass (the walks are one launch for the whole tree)."""
-        if S == 4 and which == "post":
-            return 2 + int(self.tips.kind == _lib.HX_TIPS_CODES)  # pad codes, walk, root sums
+        if S == 4 and which == "post":  # walk, root sums; outside the FP32 walks also padded codes
+            fp32_walk = code != _lib.HX_F64 and C <= 4
+            return 2 + int(self.tips.kind == _lib.HX_TIPS_CODES and not fp32_walk)
         if S == 4 and which == "pre" and code != _lib.HX_F64 and C <= 4:
             return 2  # walk, statistic reduction (mirrors use_pre_walk, csrc/layout.hpp)
         return (self.plan.post_levels if which == "post" else self.plan.pre_levels) + 1
