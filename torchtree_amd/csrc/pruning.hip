@@ -31,6 +31,7 @@
 
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 namespace hx {
@@ -230,6 +231,11 @@ static bool runs_walk4(const CallArgs& c) {
          (c.tip_kind != HX_TIPS_CODES || (size_t)c.plan->T * c.N < ((size_t)1 << 32));
 }
 
+// Whether a dense-state call's post-order runs as the walk of pruning_dwalk.hip.
+static bool runs_dwalk(const CallArgs& c) {
+  return c.dtype != HX_F64 && use_mfma(c.C, c.S, c.dtype) && c.S <= kDwalkMaxS;
+}
+
 template <typename R>
 static PassArgs<R> make_args(const CallArgs& c) {
   const WsLayout w = ws_layout(c.plan, c.S, c.N, c.C, c.K, c.dtype, c.grad_mode);
@@ -274,15 +280,26 @@ static int run_post(const CallArgs& c, double* out_l, double* out_f, double* out
   const PassArgs<R> a = make_args<R>(c);
   const hx_plan_s* plan = c.plan;
   int nparts = a.nchunks;
+  // no gradient can follow in a workspace that has no room for one (each gradient call checks for
+  // its own): then the walks need not keep the partials
+  const bool store = c.ws_bytes >= std::min(ws_layout(plan, c.S, c.N, c.C, c.K, c.dtype, 1).total,
+                                            ws_layout(plan, c.S, c.N, c.C, c.K, c.dtype, 2).total);
+  bool dwalk = false;
+  if constexpr (std::is_same<R, float>::value) {
+    if (runs_dwalk(c)) {
+      dwalk = true;
+      const int rc = launch_post_dwalk(a, plan->d_post4, plan->I, plan->post4_slots, c.tip_kind, c.S,
+                                       store, st);
+      if (rc != HX_OK) return rc;
+      nparts = a.ntiles;
+    }
+  }
   if (c.S == 4) {
     int rc = HX_OK;
     if constexpr (std::is_same<R, float>::value) {
       if (runs_walk4(c)) {
         HX_REQUIRE(dna_walk_lds(plan->T, 1, plan->walk_need, c.tip_kind, c.ncodes, 4) <= kDnaWalkLdsMax,
                    HX_ERR_UNSUPPORTED, "post-order walk: too many taxa");
-        // no gradient can follow in a workspace that has no room for one (each gradient call
-        // checks for its own): then the partials need not be kept
-        const bool store = c.ws_bytes >= ws_layout(plan, c.S, c.N, c.C, c.K, c.dtype, 2).total;
         rc = launch_post_walk4(a, plan->d_post4, plan->I, plan->post4_slots, c.tip_kind, store, st);
       } else {
         rc = launch_post_dna<R>(a, plan->d_walk, plan->I, plan->walk_need, c.tip_kind, st);
@@ -292,7 +309,7 @@ static int run_post(const CallArgs& c, double* out_l, double* out_f, double* out
     }
     if (rc != HX_OK) return rc;
     nparts = a.ntiles;
-  } else {
+  } else if (!dwalk) {
     const int H = (int)plan->post_off.size() - 1;
     for (int l = 0; l < H; ++l) {
       const int off = plan->post_off[l], width = plan->post_off[l + 1] - off;

@@ -1385,6 +1385,8 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   const int MT = S <= 16 ? 1 : (S <= 32 ? 2 : 4);
   const int threads = 2 * a.C * 64;
   const size_t lds = mfma_lds<R>(a.C, S, !post, a.tiles_per_chunk);
+  // FP32 post-orders at up to 32 states are walks (pruning_dwalk.hip)
+  HX_REQUIRE(!post || MT == 4 || sizeof(R) == 8, HX_ERR_INVALID_ARGUMENT, "dense-state post-order");
   HX_REQUIRE(lds <= 160 * 1024, HX_ERR_UNSUPPORTED, "dense-state kernel LDS exceeds 160 KiB");
   // k_pre_mfma_r addresses a (node, sample) slab of partials with 32-bit
   // element offsets, reading up to 16 C S + 64 elements past its end
@@ -1424,23 +1426,29 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   else                                                                                       \
     k_post_mfma_r<R, MTV, KVV, HX_TIPS_DENSE, SPLIT><<<grid, threads, lds_r, st>>>(a, nodes, \
                                                                                    S);
-    if (MT == 1) {
-      HX_MFR(1, 4)
-    } else if (MT == 4) {
+    if (MT == 4) {
       HX_MFR(4, 16)
-    } else if (S <= 20) {
-      HX_MFR(2, 5)
-    } else {
-      HX_MFR(2, 8)
+    } else if constexpr (sizeof(R) == 8) {
+      if (MT == 1) {
+        HX_MFR(1, 4)
+      } else if (S <= 20) {
+        HX_MFR(2, 5)
+      } else {
+        HX_MFR(2, 8)
+      }
     }
 #undef HX_MFR
   } else if (post) {
-    if (MT == 1) {
-      HX_MF_ROOT(1, 4)
-    } else if (MT == 2) {
-      if (S <= 20) { HX_MF_ROOT(2, 5) } else { HX_MF_ROOT(2, 8) }
-    } else {
+    if (MT == 4) {
       HX_MF_ROOT(4, 16)
+    } else if constexpr (sizeof(R) == 8) {
+      if (MT == 1) {
+        HX_MF_ROOT(1, 4)
+      } else if (S <= 20) {
+        HX_MF_ROOT(2, 5)
+      } else {
+        HX_MF_ROOT(2, 8)
+      }
     }
   } else if (MT == 1) {
     HX_MF_ALL(k_pre_mfma_r, 1, 4)

@@ -247,6 +247,8 @@ class Pruning:
             return 2 + int(self.tips.kind == _lib.HX_TIPS_CODES and not fp32_walk)
         if S == 4 and which == "pre" and code != _lib.HX_F64 and C <= 4:
             return 2  # walk, statistic reduction (mirrors use_pre_walk, csrc/layout.hpp)
+        if S != 4 and which == "post" and code != _lib.HX_F64 and C <= 4 and S <= 32:
+            return 2  # walk, root sums (mirrors runs_dwalk, csrc/pruning.hip)
         return (self.plan.post_levels if which == "post" else self.plan.pre_levels) + 1
 
     def forward(self, mats, freqs, props, want_root_grads=True):
