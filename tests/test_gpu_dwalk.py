@@ -28,10 +28,16 @@ CASES = [("random", 2, 1, 1, 2, False), ("caterpillar", 9, 17, 4, 3, True),
          ("random", 30, 100, 4, 32, False)]
 
 
-@pytest.mark.parametrize("shape,T,N,C,S,dense", CASES)
+# the level kernels of larger state counts: rows of a matrix and of a tile past their ends
+LEVEL_CASES = [("random", 9, 1, 1, 33, False), ("balanced", 16, 17, 4, 49, False),
+               ("random", 12, 33, 2, 61, True), ("caterpillar", 7, 150, 3, 61, False),
+               ("random", 20, 140, 4, 64, False)]
+
+
+@pytest.mark.parametrize("shape,T,N,C,S,dense", CASES + LEVEL_CASES)
 def test_dense_walks(gpu, shape, T, N, C, S, dense):
     """Tolerances: those of the other FP32 tests (logL 1e-6, gradients 1e-5 norm-wise)."""
-    print(f"case: dense FP32 walks {shape} T={T} N={N} C={C} S={S} dense={dense}", flush=True)
+    print(f"case: dense FP32 passes {shape} T={T} N={N} C={C} S={S} dense={dense}", flush=True)
     from torchtree_amd import likelihood as hl
     from torchtree_amd.serving import ResidentJob
 

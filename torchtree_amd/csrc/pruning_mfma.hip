@@ -244,6 +244,86 @@ __device__ __forceinline__ void child_row(const PassArgs<R>& a, int ch, int k, i
   }
 }
 
+// ---- FP32 rows (child partials, tips, matrices, adjoints) as they lie in memory
+//
+// An operand's lanes are patterns: loaded as operands, the lanes of a row load are rows apart and
+// each is an access of its own in the vector L1 (64 per load; it looks up about one line per clock,
+// and at 61 states these loads alone kept it busy for 96 % of the post-order with split products).
+// So rows move with lanes along the states, 64 / (16 MT) rows a load, which takes a few lines, and
+// become operands (or accumulators) through the wave's LDS tile. A coded tip's rows are the table's.
+// Rows past N (past the table: never) and states past S are out of range: they read 0 and store
+// nothing. Measured: 128 taxa x 10000 patterns, 61 states, split products: post-order 1422 -> 1104
+// us, pre-order 2715 -> 2344; FP32, 97 x 1217 at 8 samples: 1436 -> 1201, 3357 -> 3224; 20 states,
+// FP32 pre-order of 256 x 20000: 3204 -> 2990.
+constexpr unsigned kNowhere = 0x7fffff00u;
+template <int MT>
+struct NatRows {
+  static constexpr int LPR = 16 * MT, RPI = 64 / LPR, NI = kTile / RPI;  // lanes per row, rows per load
+  const float* base;         // the child's (node, sample, category) rows, or the tip table
+  bool coded;
+  int stride, N, S, lrow, bytes;  // floats between rows; the lane's first row; the table's size
+  unsigned off, step;
+  // rows of S floats, stride_ apart, N_ of them; with `codes`, the rows of a table of ncodes
+  __device__ __forceinline__ NatRows(const float* rows, int stride_, int N_, int S_, int lane,
+                                     bool codes = false, int ncodes = 0)
+      : base(rows), coded(codes), stride(stride_), N(N_), S(S_), lrow(lane / LPR),
+        bytes(ncodes * S_ * 4) {
+    const int s = lane % LPR;
+    off = s < S ? 4u * (unsigned)((coded ? 0 : lrow * stride) + s) : kNowhere;
+    step = 4u * (unsigned)(RPI * stride);
+  }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(int tile) const {
+    const int n0 = __builtin_amdgcn_readfirstlane(tile * kTile), n = min(kTile, N - n0);
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(base + (coded ? (size_t)0 : (size_t)n0 * stride)), (short)0,
+        coded ? bytes : (n > 0 ? ((n - 1) * stride + S) * 4 : 0), 0x00020000);
+  }
+  // the tile's loads I0 .. I0 + n - 1; code: of pattern tile * 16 + (lane & 15), in every lane
+  template <int n>
+  __device__ __forceinline__ void load(int tile, int i0, int code, float (&x)[n]) const {
+    const auto r = rsrc(tile);
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      unsigned o = off + (i0 + i) * step;
+      if (coded) {
+        const int cr = RPI == 1 ? __builtin_amdgcn_readlane(code, i0 + i)
+                                : __shfl(code, (i0 + i) * RPI + lrow);
+        o = off + 4u * (unsigned)(cr * S);
+      }
+      x[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)o, 0, 0));
+    }
+  }
+  // the lane's element of load i in an LDS tile of row stride LS
+  template <int LS>
+  static __device__ __forceinline__ int at(int i, int lane) {
+    return (i * RPI + lane / LPR) * LS + lane % LPR;
+  }
+  template <int LS>
+  __device__ __forceinline__ void store(int tile, const float* lt, int lane) const {
+    const auto r = rsrc(tile);
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, lt[at<LS>(i, lane)]), r,
+                                            (int)(off + i * step), 0, 0);
+  }
+};
+
+// KV words at p: 16 bytes at a time where KV allows
+template <int KV>
+__device__ __forceinline__ void lds_run(const float* p, float (&x)[KV]) {
+  if constexpr (KV % 4 == 0) {
+#pragma unroll
+    for (int q = 0; q < KV; q += 4) {
+      const vec4_t<float> v = *reinterpret_cast<const vec4_t<float>*>(p + q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[q + e] = v[e];
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < KV; ++q) x[q] = p[q];
+  }
+}
+
 // The forward product's P operand, held in registers for a chunk, and the product
 // acc[t] += L P^T over the lane's KV states g KV .. g KV + KV - 1:
 //   plain: f[t][ks] = P[16 t + nn][g KV + ks], KV steps of the 16x16x4 instruction;
@@ -268,6 +348,48 @@ struct FwdP {
       }
   }
 
+  // the same, of an FP32 matrix by way of the LDS tile lt (row stride LS) of this wave; `pt`: also
+  // the transpose's words, P[j][i] at pt[j * PS + i] (both below 4 KV)
+  template <int LS, int PS>
+  __device__ __forceinline__ void load_nat(const float* pm, int S, int lane, float* lt, float* pt) {
+    using NR = NatRows<MT>;
+    const int nn = lane & 15, g = lane >> 4;
+    const NR rows(pm, S, S, S, lane);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      float x[NR::NI], y[KV];
+      rows.load(t, 0, 0, x);
+#pragma unroll
+      for (int i = 0; i < NR::NI; ++i) {
+        lt[NR::template at<LS>(i, lane)] = x[i];
+        if (PS > 0) {
+          const int row = 16 * t + i * NR::RPI + lane / NR::LPR;
+          if (row < 4 * KV) {
+            if constexpr (SPLIT) pt[row * PS + lane % NR::LPR] = __builtin_bit_cast(float, bf_pair(x[i]));
+            else pt[row * PS + lane % NR::LPR] = x[i];
+          }
+        }
+      }
+      lds_run<KV>(lt + nn * LS + g * KV, y);
+#pragma unroll
+      for (int q = 0; q < (SPLIT ? NB * KB : KV); ++q) {
+        if constexpr (SPLIT) pack_set(b[t][q / KB], q % KB, q < KV ? y[q] : 0.f);
+        else f[t][q] = y[q];
+      }
+    }
+  }
+
+  // of the hi / lo words of split operands
+  __device__ __forceinline__ void product_words(const R (&ow)[KV], vec4_t<R> (&acc)[MT]) const {
+    BfPack<KB> ap[NB];
+#pragma unroll
+    for (int q = 0; q < NB * KB; ++q)
+      pack_set_pair(ap[q / KB], q % KB, q < KV ? __builtin_bit_cast(uint32_t, ow[q]) : 0u);
+#pragma unroll
+    for (int bb = 0; bb < NB; ++bb)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[t] = mma3(ap[bb], b[t][bb], acc[t]);
+  }
   __device__ __forceinline__ void product(const R (&arow)[KV], vec4_t<R> (&acc)[MT]) const {
     if constexpr (SPLIT) {
       BfPack<KB> ap[NB];
@@ -446,13 +568,13 @@ __global__ __launch_bounds__(512) void k_post_mfma(PassArgs<R> a,
 }
 
 // Post-order below the root (P in registers at up to 64 padded states). Every global load
-// of a tile is issued on every path so the compiler's waits are exact: child
-// rows and states are clamped to the child's own last row and state and then
-// zeroed by a multiply (every value read is a written partial), each wave
-// loads the children's scales of the tile's rows (wave 0 stages them in LDS,
-// double-buffered by tile parity so two barriers per tile suffice), and a tip
-// child's codes for the chunk are staged in LDS once. Same products as
-// k_post_mfma.
+// of a tile is issued on every path so the compiler's waits are exact: FP32 moves rows as
+// NatRows does, a tile ahead; in FP64 child rows and states are clamped to the child's own
+// last row and state and then zeroed by a select (every value read is a written partial).
+// Each wave loads the children's scales of the tile's rows (wave 0 stages them in LDS,
+// double-buffered by tile parity so two barriers per tile suffice) and a tip child's codes
+// a tile (FP32: two) ahead. Same products as k_post_mfma. What bounds it: FP32 the matrix
+// products at 8 waves per CU between barriers (29 % busy), split products the latency of a tile.
 template <typename R, int MT, int KV, int TIPS, bool SPLIT = false>
 __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
                                                      const int32_t* __restrict__ nodes, int S) {
@@ -465,7 +587,9 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
   R* Yx = reinterpret_cast<R*>(smem_raw);              // [C][16][LS] child-1 products
   R* mx = Yx + C * kTile * LS;                         // [16][4] per-row category maxima
   int* Et = reinterpret_cast<int*>(mx + 4 * kTile);    // [2 parity][2 children][16]
-  uint8_t* ctile = reinterpret_cast<uint8_t*>(Et + 4 * kTile);  // [2][tpc * 16] codes
+  // FP32: the wave's tile of child rows (its product tile, for h = 1: see the barriers)
+  constexpr bool kNat = sizeof(R) == 4;
+  R* Lt = reinterpret_cast<R*>(Et + 4 * kTile);        // [C][16][LS]
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -484,26 +608,19 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
   R* vslab = a.partials + ((size_t)(v - a.T) * a.K + k) * slab;
   const int t0 = chunk * a.tiles_per_chunk;
   const int t1 = min(t0 + a.tiles_per_chunk, a.ntiles);
-  const int npat = a.tiles_per_chunk * kTile;
 
-  if constexpr (TIPS == HX_TIPS_CODES) {
-    for (int q = threadIdx.x; q < 2 * npat; q += blockDim.x) {
-      const int hh = q >= npat, m = q - hh * npat, n = t0 * kTile + m;
-      const int chq = hh ? ch1 : ch0;
-      ctile[q] = (chq < a.T && n < a.N) ? a.codes[(size_t)chq * a.N + n] : 0;
-    }
-  }
   // categories C .. 3 of mx stay zero, so a row's maximum reads all four entries
   for (int q = threadIdx.x; q < 4 * kTile; q += blockDim.x) mx[q] = R(0);
-
+  R* lt = (kNat && h == 0 ? Lt : Yx) + (size_t)c * kTile * LS;
   FwdP<R, MT, KV, SPLIT> fp;  // P[16 t + nn][g KV + ks]
-  fp.load(a.mats + (((size_t)k * a.B + chh) * C + c) * S * S, S, nn, g);
+  const R* pm = a.mats + (((size_t)k * a.B + chh) * C + c) * S * S;
+  if constexpr (kNat) fp.template load_nat<LS, 0>(pm, S, lane, lt, nullptr);
+  else fp.load(pm, S, nn, g);
   bool stok[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) stok[t] = 16 * t + nn < S;
   const uint32_t rstep = sizeof(R) == 4 ? CS : 4 * CS;
   const uint32_t ub = (uint32_t)(acc_row<R>(g, 0) * CS + c * S + nn);
-  const uint8_t* mycodes = ctile + h * npat;
   // children's scales: lane (q = lane & 15, child (lane >> 4) & 1); a tip's reads
   // land on slab 0 of the scales and are multiplied by 0
   const int chq = ((lane >> 4) & 1) ? ch1 : ch0;
@@ -511,32 +628,16 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
   const float qmask = chq >= a.T ? 1.f : 0.f;
   lds_barrier();
 
-  // a tile's child rows, loaded as they are (rows clamped to N - 1; states past S read the
-  // row's last state, or with 16-byte loads the words after the row, which the padding after
-  // the partials keeps inside the workspace); the values past S or N are zeroed with a select
-  // when the tile starts. With split products the rows are issued one tile ahead (128 taxa,
-  // 10k patterns, 61 states: 1.79 -> 1.64 ms); the longer FP32 products hide their latency
-  // (2.01 -> 2.07 ms when issued ahead), so FP32 issues them at the tile start
-  auto post_rows = [&](int tl, R (&row)[KV]) {
+  // FP64: a tile's child rows as operands (rows clamped to N - 1, states past S read the row's
+  // last state; both are zeroed with a select when the tile starts)
+  auto post_rows = [&](int tl, int code, R (&row)[KV]) {
     const int ncl = min(tl * kTile + nn, a.N - 1);
-    if constexpr (sizeof(R) == 4 && KV % 4 == 0) {
-      if (internal) {
-        const R* rp = cslab + (uint32_t)(ncl * CS + c * S + g * KV);
-#pragma unroll
-        for (int q = 0; q < KV; q += 4) {
-          const f32x4u_t w = *reinterpret_cast<const f32x4u_t*>(rp + q);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) row[q + e] = w[e];
-        }
-        return;
-      }
-    }
     const R* bp;
     uint32_t base, last;  // first element and last state of the row read
     if (internal) {
       bp = cslab, base = (uint32_t)(ncl * CS + c * S);
     } else if constexpr (TIPS == HX_TIPS_CODES) {
-      bp = a.table, base = (uint32_t)(mycodes[(tl - t0) * kTile + nn] * S);
+      bp = a.table, base = (uint32_t)(code * S);
     } else {
       bp = a.dense + (size_t)chh * a.N * S, base = (uint32_t)(ncl * S);
     }
@@ -545,25 +646,52 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
 #pragma unroll
     for (int q = 0; q < KV; ++q) row[q] = bp[min(base + q, last)];
   };
+  // a tip's codes are on their way for the time of a tile, and so are FP32's rows
+  const bool coded = TIPS == HX_TIPS_CODES && !internal;
+  const uint8_t* tcodes = coded ? a.codes + (size_t)chh * a.N : nullptr;
+  auto code_of = [&](int tl) -> int { return coded ? tcodes[min(tl * kTile + nn, a.N - 1)] : 0; };
+  int code = code_of(t0);
   R arow[KV];
-  if constexpr (SPLIT) post_rows(t0, arow);
+  using NR = NatRows<MT>;
+  float nrow[NR::NI];
+  auto rows = [&] {
+    if constexpr (kNat)
+      return NR(internal ? cslab + c * S : (coded ? a.table : a.dense + (size_t)chh * a.N * S),
+                internal ? CS : S, a.N, S, lane, coded, a.ncodes);
+    else return 0;
+  }();
+  auto outrows = [&] {
+    if constexpr (kNat) return NR(vslab + c * S, CS, a.N, S, lane);
+    else return 0;
+  }();
+  if constexpr (kNat) {
+    rows.load(t0, 0, code, nrow);
+    code = code_of(min(t0 + 1, t1 - 1));
+  }
 
   for (int tile = t0; tile < t1; ++tile) {
     const int nbase = tile * kTile;
     const uint32_t tb = (uint32_t)nbase * (uint32_t)CS;
-    if constexpr (!SPLIT) post_rows(tile, arow);
-    {
+    if constexpr (kNat) {
+#pragma unroll
+      for (int i = 0; i < NR::NI; ++i)
+        lt[NR::template at<LS>(i, lane)] = nrow[i];
+      // (the last tile reads its own again, unused)
+      rows.load(min(tile + 1, t1 - 1), 0, code, nrow);
+      code = code_of(min(tile + 2, t1 - 1));
+      lds_run<KV>(lt + nn * LS + g * KV, arow);
+    } else {
+      post_rows(tile, code, arow);
       const bool rok = nbase + nn < a.N;
 #pragma unroll
       for (int q = 0; q < KV; ++q) arow[q] = (rok && g * KV + q < S) ? arow[q] : R(0);
+      code = code_of(min(tile + 1, t1 - 1));
     }
     const float sv = (float)sq[min(nbase + (lane & 15), a.N - 1)] * qmask;
     vec4_t<R> acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = vec4_t<R>{R(0), R(0), R(0), R(0)};
     fp.product(arow, acc);
-    // the next tile's rows (the last tile re-reads its own, unused)
-    if constexpr (SPLIT) post_rows(min(tile + 1, t1 - 1), arow);
     // lane (nn, g): acc[t][r] = Y[m = acc_row(g, r)][i = 16 t + nn]
     if (h == 1) {
 #pragma unroll
@@ -590,9 +718,6 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
     }
     lds_barrier();
     if (h == 0) {
-      const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
-          vslab + (size_t)__builtin_amdgcn_readfirstlane(nbase) * CS, (short)0,
-          kTile * CS * (int)sizeof(R), 0x00020000);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = acc_row<R>(g, r), n = nbase + m;
@@ -601,26 +726,25 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
         int e = 0;
         if (M > R(0) && isfinite(M)) frexp_(M, &e);
         const int E = et[m] + et[kTile + m] + e;
-        if (n < a.N) {
+        if constexpr (kNat) {
 #pragma unroll
-          for (int t = 0; t < MT; ++t)
-            if (stok[t]) {
-              if constexpr (sizeof(R) == 4) {
-                // a tile's rows through a descriptor at the tile: lane offset of row
-                // acc_row(g, r) in bytes, 64 t bytes as the scalar offset
-                __builtin_amdgcn_raw_buffer_store_b32(
-                    __builtin_bit_cast(uint32_t, ldexp_(x[t][r], -e)), vrs,
-                    (int)((ub + r * rstep) * (uint32_t)sizeof(R)), 64 * t, 0);
-              } else {
-                vslab[tb + ub + r * rstep + 16 * t] = ldexp_(x[t][r], -e);
-              }
-            }
+          for (int t = 0; t < MT; ++t) lt[m * LS + 16 * t + nn] = ldexp_(x[t][r], -e);
+        }
+        if (n < a.N) {
+          if constexpr (!kNat) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+              if (stok[t]) vslab[tb + ub + r * rstep + 16 * t] = ldexp_(x[t][r], -e);
+          }
           if (c == 0 && nn == 0) a.scales[((size_t)(v - a.T) * a.K + k) * a.N + n] = E;
         }
       }
     }
-    // no third barrier: h = 1 waves rewrite Yx only after the second barrier,
-    // by which the h = 0 waves have read it; mx is rewritten after the next
+    if constexpr (kNat) {
+      if (h == 0) outrows.template store<LS>(tile, lt, lane);
+    }
+    // no third barrier: h = 1 waves rewrite Yx (with the next tile's rows, or its
+    // products) only after the second barrier, by which the h = 0 waves have read it; mx is rewritten after the next
     // first barrier; Et alternates between two buffers
   }
 }
@@ -859,30 +983,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 // out-of-range ones by a multiply.
 template <typename R, int KV, int TIPS>
 __device__ __forceinline__ void pre_rows(const PassArgs<R>& a, bool internal, const R* cslab,
-                                         int chh, const uint8_t* mycodes, int tile, int t0,
-                                         int nn, int g, int S, int CS, uint32_t cb,
-                                         R (&arow)[KV]) {
+                                         int chh, int code, int tile, int nn, int g, int S, int CS,
+                                         uint32_t cb, R (&arow)[KV]) {
   const int nbase = tile * kTile;
-  if constexpr (sizeof(R) == 4 && KV % 4 == 0) {
-    // workspace rows: KV / 4 loads of 16 bytes (4-byte aligned: a category's row starts at
-    // c S floats), no clamp needed
-    if (internal) {
-      const R* rp = cslab + (uint32_t)nbase * (uint32_t)CS + cb;
-#pragma unroll
-      for (int q = 0; q < KV; q += 4) {
-        const f32x4u_t v = *reinterpret_cast<const f32x4u_t*>(rp + q);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) arow[q + e] = v[e];
-      }
-      return;
-    }
-  }
   const R* bp;
   uint32_t base, lim;
   if (internal) {
     bp = cslab, base = (uint32_t)nbase * (uint32_t)CS + cb, lim = 0xffffffffu;
   } else if constexpr (TIPS == HX_TIPS_CODES) {
-    const int code = mycodes[(tile - t0) * kTile + nn];
     bp = a.table, base = (uint32_t)(code * S + g * KV), lim = (uint32_t)(a.ncodes * S - 1);
   } else {
     bp = a.dense + (size_t)chh * a.N * S;
@@ -924,11 +1032,11 @@ constexpr int kPD = 4;
 // each tile reads them as aligned 16-byte loads from zero-padded 64 x 64 copies
 // of P and P^T (ppad). Each tile
 // issues the same global loads on every path, so the compiler's waits are
-// exact: rows past N and states past S of the workspace partials read the
-// padding that follows them, reads of caller buffers (codes, tables, dense
-// tips, weights) use clamped indices, and every such value is then zeroed.
+// exact: FP32 moves rows as NatRows does; in FP64 rows past N and states past S of the
+// workspace partials read the padding that follows them, reads of caller buffers (codes,
+// tables, dense tips, weights) use clamped indices, and every such value is then zeroed.
 // Addresses are a (node, sample) slab base plus 32-bit element offsets,
-// (n C + c) S + s. A tip child's codes for the chunk are staged in LDS once.
+// (n C + c) S + s. A tip child's codes come a tile ahead of its rows.
 // Same products and barriers as k_pre_mfma.
 template <typename R, int MT, int KV, int TIPS, bool ROOT, bool SPLIT = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
@@ -941,10 +1049,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   constexpr int KB = SSh::KB, NB = SSh::NB;
   constexpr bool kPReg = MT <= 2;
   constexpr int SP = 16 * MT;
-  // LDS row stride of the [16][SP] tiles: at 32 padded states, SP + 4 starts rows 4g + r of the
-  // accumulator layout 16g banks apart (SP puts the four lane groups g on the same banks); at 64
-  // the extra address registers would cost the kernel spills, so the tiles stay dense
-  constexpr int LS = MT <= 2 ? SP + 4 : SP;
+  // LDS row stride of the [16][SP] tiles: SP + 4 starts rows 4g + r of the accumulator layout 16g
+  // banks apart (SP puts the four lane groups g, and an operand's 16 rows, on the same banks)
+  constexpr int LS = SP + 4;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int C = a.C;
   R* Yx = reinterpret_cast<R*>(smem_raw);  // [2][C][16][LS]: P L, then Ut transposes
@@ -953,8 +1060,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   R* Lx = mxx + 8 * kTile;                 // [2][C][16][LS]: the child's partial tile
   constexpr int kPtS = SP + 1;             // row stride of the P tiles (no bank conflicts)
   R* PtL = Lx + 2 * C * kTile * LS;        // [2][C][4 KV][SP + 1]: the transpose's P (MT <= 2)
-  uint8_t* ctile = reinterpret_cast<uint8_t*>(PtL + (MT <= 2 ? 2 * C * 4 * KV * kPtS : 0));
-  // [2][tpc * 16] codes
+  R* Ux = PtL + (MT <= 2 ? 2 * C * 4 * KV * kPtS : 0);  // [C][16][LS]: the parent's adjoint (FP32)
+  constexpr bool kNat = sizeof(R) == 4;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -975,32 +1082,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   const R* pm = a.mats + (((size_t)k * a.B + chh) * C + c) * S * S;
   const int t0 = chunk * a.tiles_per_chunk;
   const int t1 = min(t0 + a.tiles_per_chunk, a.ntiles);
-  const int npat = a.tiles_per_chunk * kTile;
-
-  if constexpr (TIPS == HX_TIPS_CODES) {
-    // the chunk's codes of each tip child (0 past N)
-    for (int q = threadIdx.x; q < 2 * npat; q += blockDim.x) {
-      const int hh = q >= npat, m = q - hh * npat, n = t0 * kTile + m;
-      const int chq = hh ? ch1 : ch0;
-      ctile[q] = (chq < a.T && n < a.N) ? a.codes[(size_t)chq * a.N + n] : 0;
-    }
-  }
 
   // Pf[t][ks] = P[16 t + nn][g KV + ks] (forward), Pt[t][ks] = P[g KV + ks][16 t + nn]
   // (transpose)
   // the transpose's operand P[g KV + ks][16 t + nn] lives in this wave's LDS tile
   FwdP<R, kPReg ? MT : 1, kPReg ? KV : 1, SPLIT && kPReg> fp;
   R* ptw = PtL + (size_t)(h * C + c) * 4 * KV * kPtS;
-  if constexpr (kPReg) {
+  R* lt = Lx + (size_t)(h * C + c) * kTile * LS;  // this wave's L tile [16 patterns][LS]
+  if constexpr (kPReg && kNat) {
+    fp.template load_nat<LS, kPtS>(pm, S, lane, lt, ptw);
+  } else if constexpr (kPReg) {
     fp.load(pm, S, nn, g);
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
       for (int ks = 0; ks < KV; ++ks) {
         const int i = 16 * t + nn, j = g * KV + ks;
-        const R v = (i < S && j < S) ? pm[j * S + i] : R(0);
-        if constexpr (SPLIT) ptw[j * kPtS + i] = __builtin_bit_cast(float, bf_pair(v));
-        else ptw[j * kPtS + i] = v;
+        ptw[j * kPtS + i] = (i < S && j < S) ? pm[j * S + i] : R(0);
       }
   }
   // padded copies of P ([0]) and P^T ([1]) in lane order: lane (nn, g) finds M[16 t + nn][g KV
@@ -1026,9 +1124,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     for (int j = 0; j < MT; ++j) G[i][j] = vec4_t<R>{R(0), R(0), R(0), R(0)};
   R* mine = Yx + (size_t)(h * C + c) * kTile * LS;
   const R* other = Yx + (size_t)((1 - h) * C + c) * kTile * LS;
-  R* lt = Lx + (size_t)(h * C + c) * kTile * LS;  // this wave's L tile [16 patterns][LS]
   if (4 * KV < SP) {
-    // states 4 KV .. SP - 1 of the tile are never written
+    // states 4 KV .. SP - 1 of the tile are never written (in FP64)
     for (int q = lane; q < kTile * LS; q += 64) lt[q] = R(0);
   }
   // categories C .. 3 of dens and mxx stay zero, so sums and maxima over a
@@ -1049,16 +1146,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   const uint32_t rstep = sizeof(R) == 4 ? CS : 4 * CS;
   const uint32_t ub = (uint32_t)(acc_row<R>(g, 0) * CS + c * S + nn);
   const uint32_t cb = (uint32_t)(nn * CS + c * S + g * KV);
-  const uint8_t* mycodes = ctile + h * npat;
   lds_barrier();
   // the first tile's child rows; each tile then issues the next tile's rows
   // after its forward product, so their latency overlaps the rest of the tile
+  // (a tip's codes a tile earlier still)
+  const bool coded = TIPS == HX_TIPS_CODES && !internal;
+  const uint8_t* tcodes = coded ? a.codes + (size_t)chh * a.N : nullptr;
+  auto code_of = [&](int tl) -> int { return coded ? tcodes[min(tl * kTile + nn, a.N - 1)] : 0; };
+  int code = code_of(t0);
   R arow[KV];
-  pre_rows<R, KV, TIPS>(a, internal, cslab, chh, mycodes, t0, t0, nn, g, S, CS, cb, arow);
-  // the parent's adjoint (zero past N and S) and the weights of a tile
-  // in FP32 a tile's rows of a slab are read and written through a buffer descriptor at the
-  // tile (scalar registers), with the lane's byte offset of row acc_row(g, r) in tvo[r] and
-  // 64 t bytes as the scalar offset: no 64-bit address arithmetic per load or store
+  using NR = NatRows<MT>;
+  float nrow[NR::NI];
+  auto rows = [&] {
+    if constexpr (kNat)
+      return NR(internal ? cslab + c * S : (coded ? a.table : a.dense + (size_t)chh * a.N * S),
+                internal ? CS : S, a.N, S, lane, coded, a.ncodes);
+    else return 0;
+  }();
+  // the parent's adjoint and the child's come and go in the same way, except with split products
+  // at up to 32 states, which have no registers left for it (spills made that kernel 40 % slower):
+  // they use the accumulator layout, tvo[r] the lane's byte offset of row acc_row(g, r)
+  constexpr bool kNatU = kNat && !(kPReg && SPLIT);
   uint32_t tvo[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) tvo[r] = (ub + r * rstep) * (uint32_t)sizeof(R);
@@ -1067,84 +1175,107 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
         const_cast<R*>(sl + (size_t)__builtin_amdgcn_readfirstlane(tl * kTile) * CS), (short)0,
         kTile * CS * (int)sizeof(R), 0x00020000);
   };
-  auto load_up = [&](int tl, R (&up)[MT][4], R (&wt)[4]) {
+  // half of the rows of the parent's adjoint, which the two children's waves share through
+  // LDS; the children's rows (an internal child's adjoint takes its partial's place)
+  constexpr int NU = NR::NI / 2;
+  float un[NU];
+  auto urows = [&] {
+    if constexpr (kNat) return NR(pslab + c * S, CS, a.N, S, lane);
+    else return 0;
+  }();
+  auto crows = [&] {
+    if constexpr (kNat) return NR(cslab + c * S, CS, a.N, S, lane);
+    else return 0;
+  }();
+  R* ut = Ux + (size_t)c * kTile * LS;
+  auto load_wt = [&](int tl, R (&wt)[4]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) wt[r] = (R)a.weights[min(tl * kTile + acc_row<R>(g, r), a.N - 1)];
+  };
+  // the adjoint and the weights come a tile ahead at 64 states, so that no load from HBM is queued
+  // before the forward's P loads; below (fewer registers) with the tile
+  R wtn[4];
+  auto next_rows = [&](int tl) {
+    if constexpr (kNat) {
+      rows.load(tl, 0, code, nrow);
+      if constexpr (!ROOT && kNatU && !kPReg) urows.load(tl, h * NU, 0, un);
+      if constexpr (!kPReg) load_wt(tl, wtn);
+    } else {
+      pre_rows<R, KV, TIPS>(a, internal, cslab, chh, code, tl, nn, g, S, CS, cb, arow);
+    }
+    code = code_of(min(tl + 1, t1 - 1));
+  };
+  next_rows(t0);
+  // the parent's adjoint (zero past N and S) of a tile in the accumulator layout
+  auto load_up = [&](int tl, R (&up)[MT][4]) {
     const int nb = tl * kTile;
     const uint32_t tbl = (uint32_t)nb * (uint32_t)CS;
-    if constexpr (!ROOT && sizeof(R) == 4) {
-      const __amdgpu_buffer_rsrc_t urs = tile_rsrc(pslab, tl);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const bool ok = nb + acc_row<R>(g, r) < a.N;
+    for (int r = 0; r < 4; ++r) {
+      const bool ok = nb + acc_row<R>(g, r) < a.N;
 #pragma unroll
-        for (int t = 0; t < MT; ++t)
-          up[t][r] = __builtin_bit_cast(
-                         R, __builtin_amdgcn_raw_buffer_load_b32(urs, (int)tvo[r], 64 * t, 0)) *
+      for (int t = 0; t < MT; ++t) {
+        if constexpr (ROOT) {
+          up[t][r] = ok ? upr[t] : R(0);
+        } else if constexpr (kNat) {
+          up[t][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                   tile_rsrc(pslab, tl), (int)tvo[r], 64 * t, 0)) *
                      ((ok && stok[t]) ? R(1) : R(0));
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const bool ok = nb + acc_row<R>(g, r) < a.N;
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          if constexpr (ROOT) {
-            up[t][r] = ok ? upr[t] : R(0);
-          } else {
-            up[t][r] = pslab[tbl + ub + r * rstep + 16 * t] * ((ok && stok[t]) ? R(1) : R(0));
-          }
+        } else {
+          up[t][r] = pslab[tbl + ub + r * rstep + 16 * t] * ((ok && stok[t]) ? R(1) : R(0));
         }
       }
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) wt[r] = (R)a.weights[min(nb + acc_row<R>(g, r), a.N - 1)];
   };
-  // at 64 padded states with split products the next tile's adjoint and weights are issued
-  // with its child rows, after the forward product, so that the forward's P loads are not
-  // queued behind loads from HBM issued just before them (128 taxa, 10k patterns, 61 states:
-  // 3.30 against 3.83 ms; with FP32 products, whose longer forward hides those loads, it
-  // cost time: 4.42 against 3.86 ms)
-  constexpr bool kUpAhead = !kPReg && SPLIT;
-  R upn[MT][4], wtn[4];
-  if constexpr (kUpAhead) load_up(t0, upn, wtn);
-
   for (int tile = t0; tile < t1; ++tile) {
     const int nbase = tile * kTile;
     const uint32_t tb = (uint32_t)nbase * (uint32_t)CS;
-    pre_rows_mask<R, KV>(a.N, tile, nn, g, S, arow);
     bool rok[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) rok[r] = nbase + acc_row<R>(g, r) < a.N;
+    // the parent's adjoint and the weights (FP32: the loads of the previous tile)
     R up[MT][4], wt[4];
-    if constexpr (kUpAhead) {
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) up[t][r] = upn[t][r];
+    if constexpr (kNat && !kPReg) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) wt[r] = wtn[r];
     } else {
-      // the parent's adjoint, then the weights (the child rows were issued by the
-      // previous tile)
-      load_up(tile, up, wt);
+      load_wt(tile, wt);
+    }
+    if constexpr (kNatU && !ROOT) {
+      if constexpr (kPReg) urows.load(tile, h * NU, 0, un);
+    } else {
+      load_up(tile, up);
     }
 
     // forward P_h L_h; the tile of L is kept as the statistic's B operand
     vec4_t<R> acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = vec4_t<R>{R(0), R(0), R(0), R(0)};
+    // ow: the operand's words (values, or in the split form their BF16 pairs)
+    R ow[KV];
+    if constexpr (kNat) {
 #pragma unroll
-    for (int q = 0; q < KV; ++q) {
-      if constexpr (SPLIT) lt[nn * LS + g * KV + q] = __builtin_bit_cast(float, bf_pair(arow[q]));
-      else lt[nn * LS + g * KV + q] = arow[q];
+      for (int i = 0; i < NR::NI; ++i) {
+        R* to = lt + NR::template at<LS>(i, lane);
+        if constexpr (SPLIT) *to = __builtin_bit_cast(float, bf_pair(nrow[i]));
+        else *to = nrow[i];
+      }
+      lds_run<KV>(lt + nn * LS + g * KV, ow);
+    } else {
+      pre_rows_mask<R, KV>(a.N, tile, nn, g, S, arow);
+#pragma unroll
+      for (int q = 0; q < KV; ++q) lt[nn * LS + g * KV + q] = ow[q] = arow[q];
     }
-    if constexpr (kPReg) {
-      fp.product(arow, acc);
+    if constexpr (kPReg && !SPLIT) {
+      fp.product(ow, acc);
+    } else if constexpr (kPReg) {
+      fp.product_words(ow, acc);
     } else if constexpr (SPLIT) {
       // 64 padded states: KV = 16 = two packs of 8; blocks 4 t + 2 bb and 4 t + 2 bb + 1 of
       // the padded copy are the hi and lo operands of pack bb
       BfPack<8> ap[2];
 #pragma unroll
-      for (int q = 0; q < 16; ++q) pack_set(ap[q / 8], q % 8, arow[q]);
+      for (int q = 0; q < 16; ++q) pack_set_pair(ap[q / 8], q % 8, __builtin_bit_cast(uint32_t, ow[q]));
       PRing<kPD> ring;
       ring.start(pp4, 0);
 #pragma unroll
@@ -1165,7 +1296,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
         for (int q = 0; q < KV; q += 4) {
           const vec4_t<R> pv = __builtin_bit_cast(vec4_t<R>, ring.take(pp4, 0, 4 * t + q / 4));
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[t] = mma(arow[q + e], pv[e], acc[t]);
+          for (int e = 0; e < 4; ++e) acc[t] = mma(ow[q + e], pv[e], acc[t]);
         }
     }
 #pragma unroll
@@ -1173,10 +1304,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
       for (int r = 0; r < 4; ++r) mine[acc_row<R>(g, r) * LS + 16 * t + nn] = acc[t][r];
     // the next tile's child rows (the last tile re-reads its own, unused)
-    pre_rows<R, KV, TIPS>(a, internal, cslab, chh, mycodes, min(tile + 1, t1 - 1), t0, nn, g, S, CS,
-                          cb, arow);
-    if constexpr (kUpAhead) load_up(min(tile + 1, t1 - 1), upn, wtn);
+    if constexpr (kNatU && !ROOT) {
+#pragma unroll
+      for (int i = 0; i < NU; ++i) ut[NR::template at<LS>(h * NU + i, lane)] = un[i];
+    }
+    next_rows(min(tile + 1, t1 - 1));
     lds_barrier();
+    if constexpr (kNatU && !ROOT) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) up[t][r] = ut[acc_row<R>(g, r) * LS + 16 * t + nn];
+    }
     // Ut_h = U_p * (P_other L_other), in the accumulator layout; the row maxima
     // of Ut over (category, state) set the adjoint's rescale exponent
     R u[MT][4];
@@ -1308,7 +1447,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     // U 2^-e stays below 2 S; a power-of-two scale is exact and cancels in every
     // term of G and of the likelihood ratios below this node
     if (internal) {
-      const __amdgpu_buffer_rsrc_t crs = tile_rsrc(cslab, tile);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = acc_row<R>(g, r);
@@ -1317,16 +1455,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
         int e = 0;
         if (M > R(0) && isfinite(M)) frexp_(M, &e);
 #pragma unroll
-        for (int t = 0; t < MT; ++t)
-          if (rok[r] && stok[t]) {
-            if constexpr (sizeof(R) != 4) {
-              cslab[tb + ub + r * rstep + 16 * t] = ldexp_(nu[t][r], -e);
-            } else {
-              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ldexp_(nu[t][r], -e)),
-                                                    crs, (int)tvo[r], 64 * t, 0);
-            }
+        for (int t = 0; t < MT; ++t) {
+          const R v = ldexp_(nu[t][r], -e);
+          if constexpr (kNatU) {
+            mine[m * LS + 16 * t + nn] = v;
+          } else if (rok[r] && stok[t]) {
+            if constexpr (kNat)
+              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v),
+                                                    tile_rsrc(cslab, tile), (int)tvo[r], 64 * t, 0);
+            else
+              cslab[tb + ub + r * rstep + 16 * t] = v;
           }
+        }
       }
+      if constexpr (kNatU) crows.template store<LS>(tile, mine, lane);
     }
     // no barrier: the next tile's first barrier orders this tile's reads of
     // dens and mxx before their next writes; each wave rewrites only its own
@@ -1363,7 +1505,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 }
 
 template <typename R>
-static size_t mfma_lds(int C, int S, bool pre, int tiles_per_chunk) {
+static size_t mfma_lds(int C, int S, bool pre) {
   const int MT = S <= 16 ? 1 : (S <= 32 ? 2 : 4);
   const size_t SP = 16 * MT, rb = sizeof(R);
   // k_pre_mfma_r (MT <= 2) pads the per-row category entries to 4 and stages
@@ -1371,9 +1513,9 @@ static size_t mfma_lds(int C, int S, bool pre, int tiles_per_chunk) {
   if (pre && (MT <= 2 || rb == 4)) {
     const int KV = MT == 2 && S <= 20 ? 5 : 4 * MT;
     const size_t pt = MT <= 2 ? 2 * (size_t)C * 4 * KV * (SP + 1) : 0;  // transpose P tiles
-    // the [16][SP] tiles are stored with row stride SP + 4 at MT <= 2 (k_pre_mfma_r)
-    return (4 * C * kTile * (MT <= 2 ? SP + 4 : SP) + 12 * kTile + pt) * rb + 64 +
-           2 * (size_t)tiles_per_chunk * kTile;
+    // the [16][SP] tiles are stored with row stride SP + 4 (k_pre_mfma_r), in FP32 with one more
+    // per category (at most 88 KiB)
+    return (4 * C * kTile * (SP + 4) + 12 * kTile + pt + (rb == 4 ? C * kTile * (SP + 4) : 0)) * rb + 64;
   }
   if (pre) return (4 * C * kTile * SP + 3 * C * kTile) * rb + 64;
   return (C * kTile * SP + C * kTile) * rb + (size_t)(C * kTile + C * SP) * 8 + 3 * kTile * 4 + 64;
@@ -1384,10 +1526,18 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
                          int tips, bool root, int S, hipStream_t st) {
   const int MT = S <= 16 ? 1 : (S <= 32 ? 2 : 4);
   const int threads = 2 * a.C * 64;
-  const size_t lds = mfma_lds<R>(a.C, S, !post, a.tiles_per_chunk);
+  const size_t lds = mfma_lds<R>(a.C, S, !post);
   // FP32 post-orders at up to 32 states are walks (pruning_dwalk.hip)
   HX_REQUIRE(!post || MT == 4 || sizeof(R) == 8, HX_ERR_INVALID_ARGUMENT, "dense-state post-order");
-  HX_REQUIRE(lds <= 160 * 1024, HX_ERR_UNSUPPORTED, "dense-state kernel LDS exceeds 160 KiB");
+  // LDS holds no codes of a chunk any more, and its rows are padded at 64 states; a chunk too large
+  // for the codes stays refused
+  const size_t codes = 2 * (size_t)a.tiles_per_chunk * kTile;
+  const size_t tilef = (size_t)a.C * kTile * (16 * MT + 4);
+  const size_t pads = (sizeof(R) == 4 ? tilef * sizeof(R) : 0) +
+                      (MT == 4 ? 4 * (size_t)a.C * kTile * 4 * sizeof(R) : 0);
+  const bool pre_r = !post && (MT <= 2 || sizeof(R) == 4);
+  HX_REQUIRE(lds <= 160 * 1024 && (!pre_r || lds - pads + codes <= 160 * 1024), HX_ERR_UNSUPPORTED,
+             "dense-state kernel LDS exceeds 160 KiB");
   // k_pre_mfma_r addresses a (node, sample) slab of partials with 32-bit
   // element offsets, reading up to 16 C S + 64 elements past its end
   HX_REQUIRE((size_t)(a.N + 16) * a.C * S + 64 < ((size_t)1 << 31), HX_ERR_UNSUPPORTED,
@@ -1414,11 +1564,13 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   if (tips == HX_TIPS_CODES) HX_MF(k_post_mfma, MTV, KVV, HX_TIPS_CODES, true);              \
   else HX_MF(k_post_mfma, MTV, KVV, HX_TIPS_DENSE, true);
   if (post && !root) {
-    // scale tiles, per-row maxima, the chunk's codes
-    const size_t lds_r = (size_t)a.C * kTile * (16 * MT + 4) * sizeof(R) + 4 * kTile * sizeof(R) +
-                         4 * kTile * 4 + 2 * (size_t)a.tiles_per_chunk * kTile + 64;
-    HX_REQUIRE(lds_r <= 64 * 1024, HX_ERR_UNSUPPORTED, "dense-state post-order LDS exceeds 64 KiB");
-    // MT 4: C <= 4, so C x 16 x 64 products take at most 16 KiB (32 KiB in FP64)
+    // products, per-row maxima, scales; FP32 also the tiles of the children's rows
+    const size_t lds_b = (size_t)a.C * kTile * (16 * MT + 4) * sizeof(R) + 4 * kTile * sizeof(R) +
+                         4 * kTile * 4 + 64;
+    HX_REQUIRE(lds_b + codes <= 64 * 1024, HX_ERR_UNSUPPORTED,
+               "dense-state post-order LDS exceeds 64 KiB");
+    // (at most 36 KiB)
+    const size_t lds_r = lds_b + (sizeof(R) == 4 ? (size_t)a.C * kTile * (16 * MT + 4) * 4 : 0);
 #define HX_MFR(MTV, KVV)                                                                     \
   if (tips == HX_TIPS_CODES)                                                                 \
     k_post_mfma_r<R, MTV, KVV, HX_TIPS_CODES, SPLIT><<<grid, threads, lds_r, st>>>(a, nodes, \
