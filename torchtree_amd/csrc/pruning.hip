@@ -304,6 +304,10 @@ static int run_post(const CallArgs& c, double* out_l, double* out_f, double* out
       } else {
         rc = launch_post_dna<R>(a, plan->d_walk, plan->I, plan->walk_need, c.tip_kind, st);
       }
+    } else if (c.C <= 4) {
+      HX_REQUIRE(dna_walk_lds(plan->T, 1, plan->walk_need, c.tip_kind, c.ncodes, 8) <= kDnaWalkLdsMax,
+                 HX_ERR_UNSUPPORTED, "post-order walk: too many taxa");
+      rc = launch_post_walk64(a, plan->d_post4, plan->I, plan->post4_slots, c.tip_kind, store, st);
     } else {
       rc = launch_post_dna<R>(a, plan->d_walk, plan->I, plan->walk_need, c.tip_kind, st);
     }

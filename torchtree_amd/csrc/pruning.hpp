@@ -76,6 +76,9 @@ inline size_t dna_walk_lds(int T, int W, int need, int tips, int ncodes, size_t 
 template <typename R>
 int launch_post_dna(const PassArgs<R>& a, const int32_t* prog, int nprog, int need, int tips,
                     hipStream_t st);
+// The FP64 post-order with at most 4 categories (pruning_walk64.hip).
+int launch_post_walk64(const PassArgs<double>& a, const int32_t* prog, int nprog, int slots, int tips,
+                       bool store, hipStream_t st);
 template <typename R>
 int launch_pre_dna(const PassArgs<R>& a, const int32_t* nodes, int width, int tips, bool root,
                    hipStream_t st);

@@ -1,6 +1,7 @@
-// Four-state (nucleotide) pruning kernels on the vector units, for FP64 and for FP32 at more
-// than 4 categories (the other FP32 calls: pruning_walk.hip): one fused post-order walk of the
-// whole tree per pattern tile, and the pre-order adjoint one tree level per launch.
+// Four-state (nucleotide) pruning kernels on the vector units: one fused post-order walk of the
+// whole tree per pattern tile at more than 4 categories (FP32 and FP64; the other calls:
+// pruning_walk.hip, pruning_walk64.hip), and the pre-order adjoint one tree level per launch for
+// these and for FP64.
 //
 // Reference: calculate_treelikelihood_discrete* (torchtree/evolution/
 // tree_likelihood.py:40-278) at S = 4, where each node update is two 4x4
@@ -609,14 +610,20 @@ int launch_post_dna(const PassArgs<R>& a, const int32_t* prog, int nprog, int ne
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
     kern<<<grid, 64 * W, lds, st>>>(a, a.mats, pg, nprog, need, W);                          \
   } while (0)
-  switch (a.C) {
-    case 1: HX_WALK(1, true); break;
-    case 2: HX_WALK(2, true); break;
-    case 3: HX_WALK(4, false); break;
-    case 4: HX_WALK(4, true); break;
-    default:
-      if (a.C <= 8) HX_WALK(8, false);
-      else HX_WALK(16, false);
+  if constexpr (sizeof(R) == 4) {
+    switch (a.C) {
+      case 1: HX_WALK(1, true); break;
+      case 2: HX_WALK(2, true); break;
+      case 3: HX_WALK(4, false); break;
+      case 4: HX_WALK(4, true); break;
+      default:
+        if (a.C <= 8) HX_WALK(8, false);
+        else HX_WALK(16, false);
+    }
+  } else {
+    HX_REQUIRE(a.C > 4, HX_ERR_INVALID_ARGUMENT, "post-order walk: categories");
+    if (a.C <= 8) HX_WALK(8, false);
+    else HX_WALK(16, false);
   }
 #undef HX_WALK
   HX_HIP_TRY(hipGetLastError());

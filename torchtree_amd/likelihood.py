@@ -242,9 +242,8 @@ class Pruning:
 
     def _launches(self, which, S, C, code, K):
         """Kernel launches of one pass (the walks are one launch for the whole tree)."""
-        if S == 4 and which == "post":  # walk, root sums; outside the FP32 walks also padded codes
-            fp32_walk = code != _lib.HX_F64 and C <= 4
-            return 2 + int(self.tips.kind == _lib.HX_TIPS_CODES and not fp32_walk)
+        if S == 4 and which == "post":  # walk, root sums; past 4 categories also padded codes
+            return 2 + int(self.tips.kind == _lib.HX_TIPS_CODES and C > 4)
         if S == 4 and which == "pre" and code != _lib.HX_F64 and C <= 4:
             return 2  # walk, statistic reduction (mirrors use_pre_walk, csrc/layout.hpp)
         if S != 4 and which == "post" and code != _lib.HX_F64 and C <= 4 and S <= 32:
