@@ -1521,6 +1521,25 @@ static size_t mfma_lds(int C, int S, bool pre) {
   return (C * kTile * SP + C * kTile) * rb + (size_t)(C * kTile + C * SP) * 8 + 3 * kTile * 4 + 64;
 }
 
+// Tiles per block of a post-order level: nothing is summed over them, so it is chosen for the
+// launch. A block costs its tiles and about kSetup more (P; 0.5 and 2 were 1 % slower); blocks
+// beyond a round of the chip's 2048 waves wait for the next. With the chunks of the gradient (8
+// tiles and more at 61 states) the narrow levels near the root had 9 to 70 blocks a sample, and
+// others a nearly empty last round: 128 taxa x 10000 patterns, 61 states, split products 1104 ->
+// 968 us; FP32, 97 x 1217 at 8 samples 1201 -> 984.
+static int post_tiles(int ntiles, int C, int K, int width) {
+  constexpr double kSetup = 1.0;
+  const double slots = 256.0 * (C >= 4 ? 1 : 4 / C);
+  int best = 1;
+  double cost = 0.0;
+  for (int t = 1; t <= ntiles && t <= 64; ++t) {
+    const double blocks = (double)((ntiles + t - 1) / t) * K * width;
+    const double c = ceil(blocks / slots) * (t + kSetup);
+    if (t == 1 || c <= cost) best = t, cost = c;
+  }
+  return best;
+}
+
 template <typename R, bool SPLIT>
 static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, int width,
                          int tips, bool root, int S, hipStream_t st) {
@@ -1571,12 +1590,15 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
                "dense-state post-order LDS exceeds 64 KiB");
     // (at most 36 KiB)
     const size_t lds_r = lds_b + (sizeof(R) == 4 ? (size_t)a.C * kTile * (16 * MT + 4) * 4 : 0);
+    PassArgs<R> b = a;
+    b.tiles_per_chunk = post_tiles(a.ntiles, a.C, a.K, width);
+    grid.x = (a.ntiles + b.tiles_per_chunk - 1) / b.tiles_per_chunk;
 #define HX_MFR(MTV, KVV)                                                                     \
   if (tips == HX_TIPS_CODES)                                                                 \
-    k_post_mfma_r<R, MTV, KVV, HX_TIPS_CODES, SPLIT><<<grid, threads, lds_r, st>>>(a, nodes, \
+    k_post_mfma_r<R, MTV, KVV, HX_TIPS_CODES, SPLIT><<<grid, threads, lds_r, st>>>(b, nodes, \
                                                                                    S);       \
   else                                                                                       \
-    k_post_mfma_r<R, MTV, KVV, HX_TIPS_DENSE, SPLIT><<<grid, threads, lds_r, st>>>(a, nodes, \
+    k_post_mfma_r<R, MTV, KVV, HX_TIPS_DENSE, SPLIT><<<grid, threads, lds_r, st>>>(b, nodes, \
                                                                                    S);
     if (MT == 4) {
       HX_MFR(4, 16)
