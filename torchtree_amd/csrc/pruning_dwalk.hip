@@ -19,9 +19,11 @@
 // child back from memory and leaves the chip nearly empty at the narrow levels (about 30 us each).
 // Measured against it, 20 states, 4 categories, FP32: 256 taxa x 20000 patterns 1815 -> 1005 us,
 // 173 taxa x 3203 patterns at 8 samples 1495 -> 900 us; with split-BF16 products at the first size
-// 1747 -> 1005 us, so those calls take the FP32 products here, too. Past 32 states the operands of
-// two children's matrices no longer fit a wave's registers (61 states: 64 x 2, fetched a node ahead).
+// 1747 -> 1000 us (each operand is split when it is used; their products are those of the level
+// kernels, to the bit). Past 32 states the operands of two children's matrices no longer fit a
+// wave's registers (61 states: 64 x 2, fetched a node ahead).
 #include "pruning.hpp"
+#include "split.hpp"
 #include "walk.hpp"
 
 #include <math.h>
@@ -104,16 +106,32 @@ __device__ __forceinline__ int row_exp(const f4& mv) {
   return M > 0.f ? e : 0;
 }
 
-// acc += A B over KV steps
-template <int MT, int KV>
+// acc = A B over KV steps, on the FP32 matrix cores or as split products with the packs of the
+// level kernels (FwdP)
+template <int MT, int KV, bool SPLIT>
 __device__ __forceinline__ void product(const float (&a)[KV], const float (&b)[MT][KV], f4 (&acc)[MT]) {
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (SPLIT) {
+    constexpr int KB = SplitShape<KV>::KB;
+    static_assert(SplitShape<KV>::NB == 1, "one pack per lane");
+    BfPack<KB> ap;
 #pragma unroll
-  for (int q = 0; q < KV; ++q)
+    for (int q = 0; q < KB; ++q) pack_set(ap, q, q < KV ? a[q < KV ? q : 0] : 0.f);
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], b[t][q], acc[t], 0, 0, 0);
+    for (int t = 0; t < MT; ++t) {
+      BfPack<KB> bp;
+#pragma unroll
+      for (int q = 0; q < KB; ++q) pack_set(bp, q, q < KV ? b[t][q < KV ? q : 0] : 0.f);
+      acc[t] = mma3(ap, bp, acc[t]);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < KV; ++q)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], b[t][q], acc[t], 0, 0, 0);
+  }
 }
 
 // The lane's offsets and the operand loads of one (tile, sample, category).
@@ -217,7 +235,7 @@ static size_t post_dwalk_lds(int C, int S, int slots, int ncodes) {
 // follow). grid = ntiles * K, sample fastest, so that the blocks of one sample tend to share an
 // XCD's L2, where its P matrices are read; block = 64 C. At 3 waves per SIMD nothing spills (107
 // registers at 20 states); forced to 5 or 6 they do (256 taxa: +0 % and +55 % time).
-template <int MT, int KV, int TIPS, bool FULL, bool STORE>
+template <int MT, int KV, int TIPS, bool FULL, bool STORE, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_post_dwalk(
     PassArgs<float> a, const int* __restrict__ prog, int nprog, int slots, int S) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -325,8 +343,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     d.mask(a1);
     d.mask(a2);
     f4 y2[MT];
-    product<MT, KV>(a1, x.p1, y);
-    product<MT, KV>(a2, x.p2, y2);
+    product<MT, KV, SPLIT>(a1, x.p1, y);
+    product<MT, KV, SPLIT>(a2, x.p2, y2);
     float* m = mx + (i & 1) * kTile * 4;
 #pragma unroll
     for (int t = 0; t < MT; ++t) y[t] *= y2[t];
@@ -435,24 +453,26 @@ int launch_post_dwalk(const PassArgs<float>& a, const int32_t* prog, int nprog, 
              HX_ERR_UNSUPPORTED, "dense-state post-order LDS exceeds 64 KiB");
   const int ncodes = tips == HX_TIPS_CODES ? a.ncodes : 0;
   const unsigned grid = (unsigned)a.ntiles * (unsigned)a.K;
-#define HX_DW(MTV, KVV, FULLV)                                                                  \
-  do {                                                                                        \
-    const size_t lds = post_dwalk_lds<MTV>(a.C, S, slots, ncodes);                            \
-    auto kern = tips == HX_TIPS_CODES                                                         \
-                    ? (store ? k_post_dwalk<MTV, KVV, HX_TIPS_CODES, FULLV, true>                    \
-                             : k_post_dwalk<MTV, KVV, HX_TIPS_CODES, FULLV, false>)                  \
-                    : (store ? k_post_dwalk<MTV, KVV, HX_TIPS_DENSE, FULLV, true>                    \
-                             : k_post_dwalk<MTV, KVV, HX_TIPS_DENSE, FULLV, false>);                 \
-    if (lds > 64 * 1024)                                                                      \
-      HX_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                     \
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));  \
-    kern<<<grid, 64 * a.C, lds, st>>>(a, prog, nprog, slots, S);                              \
+#define HX_DW_K(MTV, KVV, FULLV, SPLITV)                                                     \
+  (tips == HX_TIPS_CODES ? (store ? k_post_dwalk<MTV, KVV, HX_TIPS_CODES, FULLV, true, SPLITV>    \
+                                  : k_post_dwalk<MTV, KVV, HX_TIPS_CODES, FULLV, false, SPLITV>)  \
+                         : (store ? k_post_dwalk<MTV, KVV, HX_TIPS_DENSE, FULLV, true, SPLITV>    \
+                                  : k_post_dwalk<MTV, KVV, HX_TIPS_DENSE, FULLV, false, SPLITV>))
+#define HX_DW(MTV, KVV, FULLV)                                                               \
+  do {                                                                                       \
+    const size_t lds = post_dwalk_lds<MTV>(a.C, S, slots, ncodes);                           \
+    auto kern = a.split ? HX_DW_K(MTV, KVV, FULLV, true) : HX_DW_K(MTV, KVV, FULLV, false);  \
+    if (lds > 64 * 1024)                                                                     \
+      HX_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                    \
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
+    kern<<<grid, 64 * a.C, lds, st>>>(a, prog, nprog, slots, S);                             \
   } while (0)
   if (S <= 16) HX_DW(1, 4, false);
   else if (S == 20) HX_DW(2, 5, true);
   else if (S < 20) HX_DW(2, 5, false);
   else HX_DW(2, 8, false);
 #undef HX_DW
+#undef HX_DW_K
   HX_HIP_TRY(hipGetLastError());
   return HX_OK;
 }
