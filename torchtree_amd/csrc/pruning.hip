@@ -231,6 +231,17 @@ static bool runs_walk4(const CallArgs& c) {
          (c.tip_kind != HX_TIPS_CODES || (size_t)c.plan->T * c.N < ((size_t)1 << 32));
 }
 
+// Whether a four-state FP64 call's pre-order runs as the walk of pruning_walk64.hip or by tree level. A
+// walk's chain is (0.55 + 0.19 C) us a node, whatever there is in flight (46 us for 64 taxa x 997
+// patterns at one category, 287 for 211 x 5003 at 4); a level's launch is 7 us with its gap, and a node
+// of 64 patterns 0.0025 C us more (70 and 270 + 14 gaps for the same; 64 x 100000: 858 us against 503 of
+// the walk). For one sample, since the choice may not depend on the batch: with more the walk gains.
+static bool runs_pre_walk64(const CallArgs& c) {
+  if (c.S != 4 || c.dtype != HX_F64 || c.C > 4) return false;
+  const double nodes = c.plan->I, launches = (double)c.plan->pre_off.size(), tiles = (c.N + 63) / 64;
+  return nodes * (0.55 + 0.19 * c.C) <= 7.0 * launches + 0.0025 * c.C * tiles * nodes;
+}
+
 // Whether a dense-state call's post-order runs as the walk of pruning_dwalk.hip.
 static bool runs_dwalk(const CallArgs& c) {
   return c.dtype != HX_F64 && use_mfma(c.C, c.S, c.dtype) && c.S <= kDwalkMaxS;
@@ -271,6 +282,7 @@ static PassArgs<R> make_args(const CallArgs& c) {
   a.gtau = reinterpret_cast<double*>(base + w.gpart);
   a.ppad = use_ppad(c.S, c.dtype, c.grad_mode) ? reinterpret_cast<R*>(base + w.ppad) : nullptr;
   a.split = c.dtype == HX_F32_BF16X3;
+  a.lanes = runs_pre_walk64(c);
   a.drop = runs_walk4(c) && walk_drop_mode(c.S, c.C, c.N, c.K, c.dtype, c.tip_kind) >= 0;
   return a;
 }
@@ -361,6 +373,9 @@ static int run_pre(const CallArgs& c, double* out, hipStream_t st) {
       a.nchunks = nch;
       a.gtau = reinterpret_cast<double*>(a.scales);
     }
+  }
+  if constexpr (std::is_same<R, double>::value) {
+    if (a.lanes) return launch_pre_walk64(a, plan->d_pre4, plan->I, c.tip_kind, out, st);
   }
   const int D = (int)plan->pre_off.size() - 1;
   if (a.ppad != nullptr) {

@@ -17,6 +17,7 @@ struct PassArgs {
   int ncodes;
   const R* dense;         // [T][N][S]
   R* partials;            // [I][K][N][C][S]; S = 4: [I][K][C][np][4]
+                          // (with `lanes`: [4][16] within 16 patterns)
   int32_t* scales;        // [I][K][N] (S != 4)
   uint8_t* codes_pad;     // S = 4: codes [T][ntiles * 64], rows 64-byte aligned (same memory)
   const R* freqs;
@@ -34,6 +35,7 @@ struct PassArgs {
   // Four-state FP32 walks with tip codes: the post-order stores no cherry's partial and the
   // pre-order rebuilds it from the two tips' codes.
   int drop;
+  int lanes;  // four-state FP64: partials in the lane order of the pre-order walk, which follows
 };
 
 constexpr double kLn2 = 0.69314718055994530942;
@@ -63,7 +65,7 @@ int launch_post_walk4(const PassArgs<float>& a, const int32_t* prog, int nprog, 
                       bool store, hipStream_t st);
 int launch_pre_walk4(const PassArgs<float>& a, const int32_t* prog, int nprog, int tips,
                      hipStream_t st);
-// FP64, and FP32 at more categories (pruning_dna.hip): the post-order walk on the vector units
+// More than 4 categories (pruning_dna.hip): the post-order walk on the vector units
 // and the pre-order adjoint one level per launch.
 constexpr size_t kDnaLdsBudget = 64 * 1024;
 constexpr size_t kDnaWalkLdsMax = 160 * 1024;  // gfx950 LDS per workgroup
@@ -76,9 +78,12 @@ inline size_t dna_walk_lds(int T, int W, int need, int tips, int ncodes, size_t 
 template <typename R>
 int launch_post_dna(const PassArgs<R>& a, const int32_t* prog, int nprog, int need, int tips,
                     hipStream_t st);
-// The FP64 post-order with at most 4 categories (pruning_walk64.hip).
+// FP64 with at most 4 categories: the post-order (pruning_walk64.hip).
 int launch_post_walk64(const PassArgs<double>& a, const int32_t* prog, int nprog, int slots, int tips,
                        bool store, hipStream_t st);
+// Its gradient: the pre-order and the sum of its statistics, d loglik / d mats or d tau in `out`.
+int launch_pre_walk64(const PassArgs<double>& a, const int32_t* prog, int nprog, int tips, double* out,
+                      hipStream_t st);
 template <typename R>
 int launch_pre_dna(const PassArgs<R>& a, const int32_t* nodes, int width, int tips, bool root,
                    hipStream_t st);

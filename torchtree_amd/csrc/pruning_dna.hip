@@ -1,7 +1,7 @@
 // Four-state (nucleotide) pruning kernels on the vector units: one fused post-order walk of the
 // whole tree per pattern tile at more than 4 categories (FP32 and FP64; the other calls:
 // pruning_walk.hip, pruning_walk64.hip), and the pre-order adjoint one tree level per launch for
-// these and for FP64.
+// these and for FP64 calls of few patterns on large trees.
 //
 // Reference: calculate_treelikelihood_discrete* (torchtree/evolution/
 // tree_likelihood.py:40-278) at S = 4, where each node update is two 4x4

@@ -244,8 +244,11 @@ class Pruning:
         """Kernel launches of one pass (the walks are one launch for the whole tree)."""
         if S == 4 and which == "post":  # walk, root sums; past 4 categories also padded codes
             return 2 + int(self.tips.kind == _lib.HX_TIPS_CODES and C > 4)
-        if S == 4 and which == "pre" and code != _lib.HX_F64 and C <= 4:
-            return 2  # walk, statistic reduction (mirrors use_pre_walk, csrc/layout.hpp)
+        if S == 4 and which == "pre" and C <= 4:
+            # walk, statistic reduction; or by level (mirrors runs_pre_walk64, csrc/pruning.hip)
+            nodes, tiles, levels = self.T - 1, (self.N + 63) // 64, self.plan.pre_levels + 1
+            if code != _lib.HX_F64 or nodes * (0.55 + 0.19 * C) <= 7 * levels + 0.0025 * C * tiles * nodes:
+                return 2
         if S != 4 and which == "post" and code != _lib.HX_F64 and C <= 4 and S <= 32:
             return 2  # walk, root sums (mirrors runs_dwalk, csrc/pruning.hip)
         return (self.plan.post_levels if which == "post" else self.plan.pre_levels) + 1
