@@ -284,10 +284,10 @@ def main():
         "phases_ms": {k: v["ms"] for k, v in phases.items()},
         "roofline": {
             "bound": "hbm",
-            "kernel": (("k_pre_walk (one launch, whole tree) + k_reduce_g"
+            "kernel": (("k_pre_walk4 (one launch, whole tree) + k_reduce_g"
                         if pre_walk_used(S, wl.C, 4, wl.N, wl.K) else
                         f"k_pre ({launches - 1} depth-level launches) + k_reduce_g")
-                       if dom == "preorder" else "k_post_walk (one launch, whole tree) + k_reduce_root"),
+                       if dom == "preorder" else "k_post_walk4 (one launch, whole tree) + k_reduce_root"),
             "achieved": dom_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": dom_gbs / HBM_PEAK_GBS,
             "traffic": measured_traffic(args, dom), "algorithmic_bytes": dom_b, "pass_ms": dom_ms,
             # the measured HBM bytes over the pass time, and the per-update bytes of the
