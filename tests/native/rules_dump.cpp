@@ -1,0 +1,20 @@
+// Dispatch rules of csrc/layout.hpp, for tests/test_rules.py: one query per input line.
+//   tiles S ntiles C K width f64    -> post_level_tiles
+#include <cstdio>
+#include <cstring>
+
+#include "layout.hpp"
+
+int main() {
+  char what[16];
+  while (std::scanf("%15s", what) == 1) {
+    if (!std::strcmp(what, "tiles")) {
+      int S, nt, C, K, w, f;
+      if (std::scanf("%d %d %d %d %d %d", &S, &nt, &C, &K, &w, &f) != 6) return 1;
+      std::printf("%d\n", hx::post_level_tiles(nt, S, C, K, w, f != 0));
+    } else {
+      return 1;
+    }
+  }
+  return 0;
+}

@@ -1,0 +1,46 @@
+"""The dispatch rules of csrc/layout.hpp, compiled with g++ from the library's own header."""
+import shutil
+import subprocess
+
+import pytest
+
+from torchtree_amd.build import CSRC
+
+HERE = __import__("pathlib").Path(__file__).parent
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    out = tmp_path_factory.mktemp("rules") / "rules_dump"
+    subprocess.run(["g++", "-O1", "-std=c++17", f"-I{CSRC}", f"-I{HERE.parent / 'include'}",
+                    str(HERE / "native" / "rules_dump.cpp"), "-o", str(out)], check=True)
+
+    def run(lines):
+        text = "\n".join(" ".join(map(str, ln)) for ln in lines)
+        r = subprocess.run([str(out)], input=text, capture_output=True, text=True, check=True)
+        return [int(x) for x in r.stdout.split()]
+
+    return run
+
+
+def test_post_level_tiles_cover_every_shape(ask):
+    """Always 1 .. min(ntiles, 64) tiles, whatever the shape."""
+    grid = [("tiles", S, nt, C, K, w, f) for S in (2, 16, 17, 20, 21, 32, 33, 61, 64)
+            for nt in (1, 2, 7, 63, 64, 65, 1250, 200000) for C in (1, 2, 3, 4) for K in (1, 8, 1024)
+            for w in (1, 2, 512) for f in (0, 1)]
+    got = ask(grid)
+    assert len(got) == len(grid)
+    for q, t in zip(grid, got):
+        assert 1 <= t <= min(q[2], 64), q
+
+
+@pytest.mark.parametrize("S", [2, 8, 16, 20])
+@pytest.mark.parametrize("f64", [0, 1])
+def test_post_level_tiles_leave_blocks_to_share_a_cu(ask, S, f64):
+    """Up to 20 states several blocks share a CU: a level that could give every CU eight blocks of
+    one tile gives it at least four."""
+    for nt, K, w in ((188, 8, 13), (188, 1, 64), (25, 8, 64), (1250, 1, 10)):
+        t, = ask([("tiles", S, nt, 4, K, w, f64)])
+        assert (nt + t - 1) // t * K * w >= 4 * 256, (nt, K, w, t)

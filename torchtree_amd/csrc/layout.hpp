@@ -4,6 +4,7 @@
 // host-only test drivers build it with g++ under AddressSanitizer and UBSan.
 #pragma once
 
+#include <math.h>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -107,6 +108,40 @@ inline Tiling make_tiling(int N, int C, int K, int S, int rb) {
   t.tiles_per_chunk = (t.ntiles + nch - 1) / nch;
   t.nchunks = (t.ntiles + t.tiles_per_chunk - 1) / t.tiles_per_chunk;
   return t;
+}
+
+// Tiles per block of a dense post-order level: nothing is summed over them, so it is chosen for the
+// launch, and a result does not depend on it.
+//
+// At 33 states and more a block fills a CU. It costs its tiles and about `setup` more (P, which FP64
+// loads in the lane order of its operand), and blocks beyond a round of the chip wait for the next:
+// in the chunks of the gradient (8 tiles and more) the narrow levels near the root had 9 to 70 blocks
+// a sample, and others a nearly empty last round (61 states, 128 taxa x 10000 patterns, split
+// products: 1104 -> 968 us; FP32, 97 x 1217 at 8 samples: 1201 -> 984).
+//
+// Below, blocks share a CU and hide each other's latency, and rounds of one block per CU leave it
+// idle. There a level takes about (blocks / 256 + tail) (t + set-up), least at t ~ sqrt(tiles C) with
+// a factor that grows with the set-up. Against every t of 1 to 16 on all levels, at 2, 8, 20 and 27
+// states, 50 taxa x 100 patterns to 128 x 100000, 1 to 16 samples, this is 10 % behind the best of
+// them at most and mostly ahead; rounds of one block per CU were 0 to 73 % behind. FP64, 2 states, 4
+// categories, 50 taxa x 3000 patterns at 8 samples: 570 us in such rounds, 348 in the gradient's
+// chunks, 333 now; 20 states, 128 x 20000: 1773 in such rounds, 1556 now.
+inline int post_level_tiles(int ntiles, int S, int C, int K, int width, bool f64) {
+  if (S <= 32) {
+    const double q = S <= 16 ? 4096.0 : (S <= 20 && C <= 2 ? 2048.0 : 1024.0);
+    const double t = sqrt((double)ntiles * K * width * C / q);
+    const int nch = (int)(ntiles / (t < 1.0 ? 1.0 : t) + 0.5), least = (ntiles + 63) / 64;
+    return (ntiles + (nch > least ? nch : least) - 1) / (nch > least ? nch : least);  // even chunks
+  }
+  const double setup = f64 ? 4.0 : 1.0, slots = 256.0 * (C >= 4 ? 1 : 4 / C);
+  int best = 1;
+  double cost = 0.0;
+  for (int t = 1; t <= ntiles && t <= 64; ++t) {
+    const double blocks = (double)((ntiles + t - 1) / t) * K * width;
+    const double c = ceil(blocks / slots) * (t + setup);
+    if (t == 1 || c <= cost) best = t, cost = c;
+  }
+  return best;
 }
 
 // FP32 gradients at 33..64 states read P and P^T from zero-padded 64 x 64 copies.

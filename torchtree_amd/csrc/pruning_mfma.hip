@@ -1448,26 +1448,6 @@ static size_t mfma_lds(int C, int S, bool pre) {
   return (C * kTile * SP + C * kTile) * rb + (size_t)(C * kTile + C * SP) * 8 + 3 * kTile * 4 + 64;
 }
 
-// Tiles per block of a post-order level: nothing is summed over them, so it is chosen for the
-// launch. A block costs its tiles and about kSetup more (P, which FP64 loads in the lane order of its
-// operand; FP32 with 0.5 and 2: 1 % slower; FP64 amino acids, 39 taxa x 40000 patterns, with 2 and
-// 4: 1354 and 1194 us, 1251 in the gradient's chunks; x 1111: 93 either way, 190 there); blocks beyond a round of the chip's 2048 waves wait for the next. With the chunks of the gradient (8
-// tiles and more at 61 states) the narrow levels near the root had 9 to 70 blocks a sample, and
-// others a nearly empty last round: 128 taxa x 10000 patterns, 61 states, split products 1104 ->
-// 968 us; FP32, 97 x 1217 at 8 samples 1201 -> 984.
-static int post_tiles(int ntiles, int C, int K, int width, bool f64) {
-  const double kSetup = f64 ? 4.0 : 1.0;
-  const double slots = 256.0 * (C >= 4 ? 1 : 4 / C);
-  int best = 1;
-  double cost = 0.0;
-  for (int t = 1; t <= ntiles && t <= 64; ++t) {
-    const double blocks = (double)((ntiles + t - 1) / t) * K * width;
-    const double c = ceil(blocks / slots) * (t + kSetup);
-    if (t == 1 || c <= cost) best = t, cost = c;
-  }
-  return best;
-}
-
 template <typename R, bool SPLIT>
 static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, int width,
                          int tips, bool root, int S, hipStream_t st) {
@@ -1519,7 +1499,7 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
     // (at most 36 KiB)
     const size_t lds_r = lds_b + (sizeof(R) == 4 ? (size_t)a.C * kTile * (16 * MT + 4) * 4 : 0);
     PassArgs<R> b = a;
-    b.tiles_per_chunk = post_tiles(a.ntiles, a.C, a.K, width, sizeof(R) == 8);
+    b.tiles_per_chunk = post_level_tiles(a.ntiles, S, a.C, a.K, width, sizeof(R) == 8);
     grid.x = (a.ntiles + b.tiles_per_chunk - 1) / b.tiles_per_chunk;
 #define HX_MFR(MTV, KVV)                                                                     \
   if (tips == HX_TIPS_CODES)                                                                 \
