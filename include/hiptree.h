@@ -94,6 +94,11 @@ int hx_plan_info(hx_plan_t plan, int* post_levels, int* pre_levels, int* max_wid
 int hx_plan_walk_info(hx_plan_t plan, int* post_need, int* pre_depth, int* cherries,
                       int* dropped_mode0, int* dropped_mode1);
 
+/* Kernel launches of one pass of such a call (no reference counterpart: accounting): of hx_loglik
+ * (grad_mode HX_GRAD_NONE), hx_loglik_grad_mats or hx_loglik_grad_tau. 0 for invalid arguments. */
+int hx_pass_launches(hx_plan_t plan, int S, int N, int C, int K, int dtype, int tip_kind,
+                     int grad_mode);
+
 /* Device workspace for one call. grad_mode: HX_GRAD_NONE (hx_loglik only),
  * HX_GRAD_MATS (then hx_loglik_grad_mats), HX_GRAD_TAU (then hx_loglik_grad_tau). */
 enum { HX_GRAD_NONE = 0, HX_GRAD_MATS = 1, HX_GRAD_TAU = 2 };

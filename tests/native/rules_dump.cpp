@@ -1,5 +1,6 @@
 // Dispatch rules of csrc/layout.hpp, for tests/test_rules.py: one query per input line.
 //   tiles S ntiles C K width f64    -> post_level_tiles
+//   dwalk S C I levels ntiles K     -> use_dwalk
 #include <cstdio>
 #include <cstring>
 
@@ -12,6 +13,10 @@ int main() {
       int S, nt, C, K, w, f;
       if (std::scanf("%d %d %d %d %d %d", &S, &nt, &C, &K, &w, &f) != 6) return 1;
       std::printf("%d\n", hx::post_level_tiles(nt, S, C, K, w, f != 0));
+    } else if (!std::strcmp(what, "dwalk")) {
+      int S, C, I, h, nt, K;
+      if (std::scanf("%d %d %d %d %d %d", &S, &C, &I, &h, &nt, &K) != 6) return 1;
+      std::printf("%d\n", (int)hx::use_dwalk(S, C, I, h, nt, K));
     } else {
       return 1;
     }

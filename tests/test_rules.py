@@ -44,3 +44,12 @@ def test_post_level_tiles_leave_blocks_to_share_a_cu(ask, S, f64):
     for nt, K, w in ((188, 8, 13), (188, 1, 64), (25, 8, 64), (1250, 1, 10)):
         t, = ask([("tiles", S, nt, 4, K, w, f64)])
         assert (nt + t - 1) // t * K * w >= 4 * 256, (nt, K, w, t)
+
+
+@pytest.mark.parametrize("S", [2, 8, 16, 18, 20, 27, 32])
+@pytest.mark.parametrize("C", [1, 2, 3, 4])
+def test_dense_walk_only_where_its_chain_is_hidden(ask, S, C):
+    """A walk's time at few patterns is the chain of all its nodes, a level's a launch: few patterns
+    on a bushy tree go by level, a caterpillar walks; past 32 states there is no walk."""
+    assert ask([("dwalk", S, C, 127, 7, 1, 1), ("dwalk", S, C, 349, 18, 4, 1),
+                ("dwalk", S, C, 199, 199, 1, 1), ("dwalk", 33, C, 199, 199, 1, 1)]) == [0, 0, 1, 0]

@@ -144,6 +144,32 @@ inline int post_level_tiles(int ntiles, int S, int C, int K, int width, bool f64
   return best;
 }
 
+// Whether a dense FP32 or split-BF16 post-order runs as one walk of the tree (pruning_dwalk.hip) or
+// by level (k_post_mfma_r). Both leave the same partials and root sums to the bit, so the choice may
+// depend on the batch. Times in us, B blocks = tiles x samples, I internal nodes:
+//   walk   8 + I (a + b C max(0, B - 256)): a node's chain a, whatever there is in flight up to a
+//          block per CU, then the blocks' work. The states decide how P comes (pruning_dwalk.hip):
+//          20 in 16-byte loads, the other sizes word by word, and rows of a multiple of 8 states
+//          (past 20; of 16 with several categories) fall on the same banks.
+//   levels (launch) x levels + I B C v.
+// Measured at 15 state counts of 2 to 32, 1 to 4 categories, 8 to 350 taxa (caterpillars to balanced
+// trees), 1 to 100000 patterns and 1 to 32 samples, 7092 calls: the faster one is chosen but for
+// 65 that lose 10 to 42 %; with the walk everywhere 350 taxa x 60 patterns, 27 states, 4 categories
+// took 1068 us (levels 112), 128 x 400 at 20 states 163 (60).
+constexpr int kDwalkMaxS = 32;
+inline bool use_dwalk(int S, int C, int I, int levels, int ntiles, int K) {
+  if (S > kDwalkMaxS) return false;
+  const double blocks = (double)ntiles * K, past = blocks > 256 ? blocks - 256 : 0;
+  double a, b;
+  if (S <= 16) a = 0.73 + 0.08 * C, b = S == 16 && C > 1 ? 0.001 : 0.0005;
+  else if (S < 20) a = 0.8 + 0.27 * C, b = 0.0009;
+  else if (S == 20) a = 0.84 + 0.1 * C, b = 0.0006;
+  else a = 0.95 + 0.47 * C, b = S % 8 == 0 ? 0.003 : 0.0019;
+  const double launch = S <= 16 ? 4.25 + 0.1 * C : 4.7 + 0.22 * C;
+  const double v = S <= 16 ? 0.00067 : (S <= 20 ? 0.00115 : 0.0016);
+  return 8 + I * (a + b * C * past) <= levels * launch + I * blocks * C * v;
+}
+
 // FP32 gradients at 33..64 states read P and P^T from zero-padded 64 x 64 copies.
 inline bool use_ppad(int S, int dtype, int grad_mode) {
   return grad_mode != 0 && dtype != HX_F64 && S > 32 && S <= 64;

@@ -244,7 +244,8 @@ static bool runs_pre_walk64(const CallArgs& c) {
 
 // Whether a dense-state call's post-order runs as the walk of pruning_dwalk.hip.
 static bool runs_dwalk(const CallArgs& c) {
-  return c.dtype != HX_F64 && use_mfma(c.C, c.S, c.dtype) && c.S <= kDwalkMaxS;
+  return c.dtype != HX_F64 && use_mfma(c.C, c.S, c.dtype) &&
+         use_dwalk(c.S, c.C, c.plan->I, (int)c.plan->post_off.size() - 1, (c.N + 15) / 16, c.K);
 }
 
 template <typename R>
@@ -327,10 +328,12 @@ static int run_post(const CallArgs& c, double* out_l, double* out_f, double* out
     nparts = a.ntiles;
   } else if (!dwalk) {
     // the root alone, in at most 512 parts of its own (there is room for one per tile): in the
-    // gradient's chunks its 9 to 128 blocks a sample took 84 to 99 us at 61 states
+    // gradient's chunks its 9 to 128 blocks a sample took 84 to 99 us at 61 states. Where a walk may
+    // take the call at another batch size, a part per tile, as there: the same sums
     PassArgs<R> root = a;
     if (use_mfma(c.C, c.S, c.dtype)) {
-      root.tiles_per_chunk = (a.ntiles + 511) / 512;
+      const bool walks = c.dtype != HX_F64 && c.S <= kDwalkMaxS;
+      root.tiles_per_chunk = walks ? 1 : (a.ntiles + 511) / 512;
       root.nchunks = nparts = (a.ntiles + root.tiles_per_chunk - 1) / root.tiles_per_chunk;
     }
     const int H = (int)plan->post_off.size() - 1;
@@ -414,6 +417,20 @@ static int run_pre(const CallArgs& c, double* out, hipStream_t st) {
 }  // namespace hx
 
 extern "C" {
+
+int hx_pass_launches(hx_plan_t plan, int S, int N, int C, int K, int dtype, int tip_kind,
+                     int grad_mode) {
+  if (!plan || S < 2 || N < 1 || C < 1 || K < 1 || !hx::dtype_ok(dtype)) return 0;
+  hx::CallArgs c{};
+  c.plan = plan, c.S = S, c.N = N, c.C = C, c.K = K, c.dtype = dtype, c.tip_kind = tip_kind;
+  const bool pre = grad_mode != HX_GRAD_NONE;
+  if (S == 4 && (hx::runs_walk4(c) || (pre ? hx::runs_pre_walk64(c) : dtype == HX_F64 && C <= 4)))
+    return 2;  // walk, sums
+  if (S == 4 && !pre) return 2 + (tip_kind == HX_TIPS_CODES);  // padded codes, walk, sums
+  if (!pre && hx::runs_dwalk(c)) return 2;
+  const int levels = (int)(pre ? plan->pre_off.size() : plan->post_off.size()) - 1;
+  return levels + 1 + hx::use_ppad(S, dtype, grad_mode);  // (padded copies of P,) levels, sums
+}
 
 size_t hx_workspace_bytes(hx_plan_t plan, int S, int N, int C, int K, int dtype, int grad_mode) {
   if (!plan || grad_mode < 0 || grad_mode > 2) return 0;

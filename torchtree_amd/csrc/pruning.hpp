@@ -89,8 +89,7 @@ int launch_pre_dna(const PassArgs<R>& a, const int32_t* nodes, int width, int ti
                    hipStream_t st);
 
 // Dense states as walks (pruning_dwalk.hip): FP32 and split-BF16 calls at up to kDwalkMaxS states
-// and 4 categories. `store`: keep the partials for a gradient.
-constexpr int kDwalkMaxS = 32;
+// and 4 categories (use_dwalk in layout.hpp). `store`: keep the partials for a gradient.
 int launch_post_dwalk(const PassArgs<float>& a, const int32_t* prog, int nprog, int slots, int tips,
                       int S, bool store, hipStream_t st);
 

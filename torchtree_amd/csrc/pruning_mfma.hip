@@ -1454,8 +1454,6 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   const int MT = S <= 16 ? 1 : (S <= 32 ? 2 : 4);
   const int threads = 2 * a.C * 64;
   const size_t lds = mfma_lds<R>(a.C, S, !post);
-  // FP32 post-orders at up to 32 states are walks (pruning_dwalk.hip)
-  HX_REQUIRE(!post || MT == 4 || sizeof(R) == 8, HX_ERR_INVALID_ARGUMENT, "dense-state post-order");
   // LDS holds no codes of a chunk any more, and its rows are padded at 64 states; a chunk too large
   // for the codes stays refused
   const size_t codes = 2 * (size_t)a.tiles_per_chunk * kTile;
@@ -1508,29 +1506,23 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   else                                                                                       \
     k_post_mfma_r<R, MTV, KVV, HX_TIPS_DENSE, SPLIT><<<grid, threads, lds_r, st>>>(b, nodes, \
                                                                                    S);
-    if (MT == 4) {
+    if (MT == 1) {
+      HX_MFR(1, 4)
+    } else if (MT == 4) {
       HX_MFR(4, 16)
-    } else if constexpr (sizeof(R) == 8) {
-      if (MT == 1) {
-        HX_MFR(1, 4)
-      } else if (S <= 20) {
-        HX_MFR(2, 5)
-      } else {
-        HX_MFR(2, 8)
-      }
+    } else if (S <= 20) {
+      HX_MFR(2, 5)
+    } else {
+      HX_MFR(2, 8)
     }
 #undef HX_MFR
   } else if (post) {
-    if (MT == 4) {
+    if (MT == 1) {
+      HX_MF_ROOT(1, 4)
+    } else if (MT == 2) {
+      if (S <= 20) { HX_MF_ROOT(2, 5) } else { HX_MF_ROOT(2, 8) }
+    } else {
       HX_MF_ROOT(4, 16)
-    } else if constexpr (sizeof(R) == 8) {
-      if (MT == 1) {
-        HX_MF_ROOT(1, 4)
-      } else if (S <= 20) {
-        HX_MF_ROOT(2, 5)
-      } else {
-        HX_MF_ROOT(2, 8)
-      }
     }
   } else if (MT == 1) {
     HX_MF_ALL(k_pre_mfma_r, 1, 4)

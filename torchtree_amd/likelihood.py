@@ -240,18 +240,10 @@ class Pruning:
             tips_p, table_p = self.tips.dense_as(dtype), None
         return K, B, C, S, code, tips_p, table_p
 
-    def _launches(self, which, S, C, code, K):
-        """Kernel launches of one pass (the walks are one launch for the whole tree)."""
-        if S == 4 and which == "post":  # walk, root sums; past 4 categories also padded codes
-            return 2 + int(self.tips.kind == _lib.HX_TIPS_CODES and C > 4)
-        if S == 4 and which == "pre" and C <= 4:
-            # walk, statistic reduction; or by level (mirrors runs_pre_walk64, csrc/pruning.hip)
-            nodes, tiles, levels = self.T - 1, (self.N + 63) // 64, self.plan.pre_levels + 1
-            if code != _lib.HX_F64 or nodes * (0.55 + 0.19 * C) <= 7 * levels + 0.0025 * C * tiles * nodes:
-                return 2
-        if S != 4 and which == "post" and code != _lib.HX_F64 and C <= 4 and S <= 32:
-            return 2  # walk, root sums (mirrors runs_dwalk, csrc/pruning.hip)
-        return (self.plan.post_levels if which == "post" else self.plan.pre_levels) + 1
+    def _launches(self, grad_mode, S, C, code, K):
+        """Kernel launches of one pass."""
+        return _lib.load().hx_pass_launches(self.plan.handle, S, self.N, C, K, code, self.tips.kind,
+                                            grad_mode)
 
     def forward(self, mats, freqs, props, want_root_grads=True):
         """mats [K,B,C,S,S]; freqs [K|1,S]; props [K|1,C] (all the same dtype, contiguous).
@@ -268,7 +260,7 @@ class Pruning:
         out = torch.empty(K, dtype=torch.float64, device=dev)
         dfreqs = torch.empty(K, S, dtype=torch.float64, device=dev) if want_root_grads else None
         dprops = torch.empty(K, C, dtype=torch.float64, device=dev) if want_root_grads else None
-        with timing.phase("postorder", self._launches("post", S, C, code, K)):
+        with timing.phase("postorder", self._launches(_lib.HX_GRAD_NONE, S, C, code, K)):
             rc = lib.hx_loglik(
             self.plan.handle, S, self.N, C, K, code, self.tips.kind,
             _lib.ptr(tips_p), _lib.ptr(table_p), self.tips.ncodes,
@@ -287,7 +279,7 @@ class Pruning:
         K, B, C, S, code, tips_p, table_p = self._common(mats, freqs, props, dtype)
         dev = mats.device
         dmats = torch.empty(K, B, C, S, S, dtype=torch.float64, device=dev)
-        with timing.phase("preorder", self._launches("pre", S, C, code, K)):
+        with timing.phase("preorder", self._launches(_lib.HX_GRAD_MATS, S, C, code, K)):
             rc = lib.hx_loglik_grad_mats(
             self.plan.handle, S, self.N, C, K, code, self.tips.kind,
             _lib.ptr(tips_p), _lib.ptr(table_p), self.tips.ncodes,
