@@ -144,6 +144,18 @@ inline int post_level_tiles(int ntiles, int S, int C, int K, int width, bool f64
   return best;
 }
 
+// Whether the FP32 level kernels move rows with lanes along the states (NatRows) or load them as
+// operands, a lane per pattern. Up to 12 states, and up to 20 with few categories, rows are short:
+// most lanes of a row load idle, and an operand load takes few lines. Operands against rows, the
+// post- and the pre-order of 50 to 350 taxa x 60 to 20000 patterns: 2 and 8 states 0.80 to 1.02 and
+// 0.84 to 1.05 (split products to 1.15, at 3000 patterns x 8 samples), 18 and 20 states with 1 to 3
+// categories 0.80 to 1.21 and 0.87 to 1.05 (the larger ones at sizes that walk), with 4 0.99 to 1.29
+// and 1.02 to 1.12; 16 states with several categories 0.94 to 1.24 and 0.91 to 1.26; 27 states 0.88
+// to 1.10 and 0.95 to 1.11, 32 0.96 to 1.66 and 0.98 to 1.40.
+inline bool use_nat_rows(int S, int C) {
+  return S > 20 || (S > 16 ? C >= 4 : S > 12 && C >= 2);
+}
+
 // Whether a dense FP32 or split-BF16 post-order runs as one walk of the tree (pruning_dwalk.hip) or
 // by level (k_post_mfma_r). Both leave the same partials and root sums to the bit, so the choice may
 // depend on the batch. Times in us, B blocks = tiles x samples, I internal nodes:

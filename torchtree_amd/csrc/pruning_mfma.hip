@@ -179,9 +179,10 @@ __device__ __forceinline__ void child_row(const PassArgs<R>& a, int ch, int k, i
 // So rows move with lanes along the states, 64 / (16 MT) rows a load, which takes a few lines, and
 // become operands (or accumulators) through the wave's LDS tile. A coded tip's rows are the table's.
 // Rows past N (past the table: never) and states past S are out of range: they read 0 and store
-// nothing. Measured: 128 taxa x 10000 patterns, 61 states, split products: post-order 1422 -> 1104
-// us, pre-order 2715 -> 2344; FP32, 97 x 1217 at 8 samples: 1436 -> 1201, 3357 -> 3224; 20 states,
-// FP32 pre-order of 256 x 20000: 3204 -> 2990.
+// nothing. Fewer states leave most lanes of such a load idle and gain nothing: use_nat_rows
+// (layout.hpp). Measured: 128 taxa x 10000 patterns, 61 states, split products: post-order 1422 -> 1104
+// us, pre-order 2715 -> 2344; FP32, 97 x 1217 at 8 samples: 1436 -> 1201, 3357 -> 3224; 20 states, 4
+// categories, FP32 pre-order of 256 x 20000: 3204 -> 2990.
 constexpr unsigned kNowhere = 0x7fffff00u;
 template <int MT>
 struct NatRows {
@@ -495,14 +496,14 @@ __global__ __launch_bounds__(512) void k_post_mfma(PassArgs<R> a,
 }
 
 // Post-order below the root (P in registers at up to 64 padded states). Every global load
-// of a tile is issued on every path so the compiler's waits are exact: FP32 moves rows as
-// NatRows does, a tile ahead; in FP64 child rows and states are clamped to the child's own
+// of a tile is issued on every path so the compiler's waits are exact: with NAT, rows move as
+// in NatRows, a tile ahead; otherwise child rows and states are clamped to the child's own
 // last row and state and then zeroed by a select (every value read is a written partial).
 // Each wave loads the children's scales of the tile's rows (wave 0 stages them in LDS,
 // double-buffered by tile parity so two barriers per tile suffice) and a tip child's codes
-// a tile (FP32: two) ahead. Same products as k_post_mfma. What bounds it: FP32 the matrix
+// a tile (NAT: two) ahead. Same products as k_post_mfma. What bounds it: FP32 the matrix
 // products at 8 waves per CU between barriers (29 % busy), split products the latency of a tile.
-template <typename R, int MT, int KV, int TIPS, bool SPLIT = false>
+template <typename R, int MT, int KV, int TIPS, bool SPLIT, bool NAT>
 __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
                                                      const int32_t* __restrict__ nodes, int S) {
   constexpr int SP = 16 * MT;
@@ -515,7 +516,7 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
   R* mx = Yx + C * kTile * LS;                         // [16][4] per-row category maxima
   int* Et = reinterpret_cast<int*>(mx + 4 * kTile);    // [2 parity][2 children][16]
   // FP32: the wave's tile of child rows (its product tile, for h = 1: see the barriers)
-  constexpr bool kNat = sizeof(R) == 4;
+  constexpr bool kNat = NAT;
   R* Lt = reinterpret_cast<R*>(Et + 4 * kTile);        // [C][16][LS]
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -559,6 +560,18 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
   // last state; both are zeroed with a select when the tile starts)
   auto post_rows = [&](int tl, int code, R (&row)[KV]) {
     const int ncl = min(tl * kTile + nn, a.N - 1);
+    if constexpr (sizeof(R) == 4 && KV % 4 == 0) {
+      if (internal) {  // (the words after a row are inside the workspace)
+        const R* rp = cslab + (uint32_t)(ncl * CS + c * S + g * KV);
+#pragma unroll
+        for (int q = 0; q < KV; q += 4) {
+          const f32x4u_t w = *reinterpret_cast<const f32x4u_t*>(rp + q);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) row[q + e] = w[e];
+        }
+        return;
+      }
+    }
     const R* bp;
     uint32_t base, last;  // first element and last state of the row read
     if (internal) {
@@ -913,6 +926,20 @@ __device__ __forceinline__ void pre_rows(const PassArgs<R>& a, bool internal, co
                                          int chh, int code, int tile, int nn, int g, int S, int CS,
                                          uint32_t cb, R (&arow)[KV]) {
   const int nbase = tile * kTile;
+  if constexpr (sizeof(R) == 4 && KV % 4 == 0) {
+    // workspace rows: KV / 4 loads of 16 bytes (4-byte aligned: a category's row starts at
+    // c S floats)
+    if (internal) {
+      const R* rp = cslab + (uint32_t)nbase * (uint32_t)CS + cb;
+#pragma unroll
+      for (int q = 0; q < KV; q += 4) {
+        const f32x4u_t v = *reinterpret_cast<const f32x4u_t*>(rp + q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) arow[q + e] = v[e];
+      }
+      return;
+    }
+  }
   const R* bp;
   uint32_t base, lim;
   if (internal) {
@@ -959,13 +986,13 @@ constexpr int kPD = 4;
 // each tile reads them as aligned 16-byte loads from zero-padded 64 x 64 copies
 // of P and P^T (ppad). Each tile
 // issues the same global loads on every path, so the compiler's waits are
-// exact: FP32 moves rows as NatRows does; in FP64 rows past N and states past S of the
+// exact: with NAT, rows move as in NatRows; otherwise rows past N and states past S of the
 // workspace partials read the padding that follows them, reads of caller buffers (codes,
 // tables, dense tips, weights) use clamped indices, and every such value is then zeroed.
 // Addresses are a (node, sample) slab base plus 32-bit element offsets,
 // (n C + c) S + s. A tip child's codes come a tile ahead of its rows.
 // Same products and barriers as k_pre_mfma.
-template <typename R, int MT, int KV, int TIPS, bool ROOT, bool SPLIT = false>
+template <typename R, int MT, int KV, int TIPS, bool ROOT, bool SPLIT, bool NAT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     sizeof(R) == 4 && MT <= 2 ? (SPLIT && KV == 8 ? 3 : 4) : 1))) void k_pre_mfma_r(
     PassArgs<R> a, const int32_t* __restrict__ nodes, int S) {
@@ -988,7 +1015,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   constexpr int kPtS = SP + 1;             // row stride of the P tiles (no bank conflicts)
   R* PtL = Lx + 2 * C * kTile * LS;        // [2][C][4 KV][SP + 1]: the transpose's P (MT <= 2)
   R* Ux = PtL + (MT <= 2 ? 2 * C * 4 * KV * kPtS : 0);  // [C][16][LS]: the parent's adjoint (FP32)
-  constexpr bool kNat = sizeof(R) == 4;
+  constexpr bool kNat = NAT;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -1025,7 +1052,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
       for (int ks = 0; ks < KV; ++ks) {
         const int i = 16 * t + nn, j = g * KV + ks;
-        ptw[j * kPtS + i] = (i < S && j < S) ? pm[j * S + i] : R(0);
+        const R v = (i < S && j < S) ? pm[j * S + i] : R(0);
+        if constexpr (SPLIT) ptw[j * kPtS + i] = __builtin_bit_cast(float, bf_pair(v));
+        else ptw[j * kPtS + i] = v;
       }
   }
   // padded copies of P ([0]) and P^T ([1]) in lane order: lane (nn, g) finds M[16 t + nn][g KV
@@ -1052,7 +1081,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   R* mine = Yx + (size_t)(h * C + c) * kTile * LS;
   const R* other = Yx + (size_t)((1 - h) * C + c) * kTile * LS;
   if (4 * KV < SP) {
-    // states 4 KV .. SP - 1 of the tile are never written (in FP64)
+    // states 4 KV .. SP - 1 of the tile are never written (as operands)
     for (int q = lane; q < kTile * LS; q += 64) lt[q] = R(0);
   }
   // categories C .. 3 of dens and mxx stay zero, so sums and maxima over a
@@ -1144,12 +1173,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
       for (int t = 0; t < MT; ++t) {
         if constexpr (ROOT) {
           up[t][r] = ok ? upr[t] : R(0);
-        } else if constexpr (kNat) {
-          up[t][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                   tile_rsrc(pslab, tl), (int)tvo[r], 64 * t, 0)) *
-                     ((ok && stok[t]) ? R(1) : R(0));
         } else {
-          up[t][r] = pslab[tbl + ub + r * rstep + 16 * t] * ((ok && stok[t]) ? R(1) : R(0));
+          R v;
+          if constexpr (sizeof(R) == 4)
+            v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                              tile_rsrc(pslab, tl), (int)tvo[r], 64 * t, 0));
+          else v = pslab[tbl + ub + r * rstep + 16 * t];
+          up[t][r] = v * ((ok && stok[t]) ? R(1) : R(0));
         }
       }
     }
@@ -1191,7 +1221,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     } else {
       pre_rows_mask<R, KV>(a.N, tile, nn, g, S, arow);
 #pragma unroll
-      for (int q = 0; q < KV; ++q) lt[nn * LS + g * KV + q] = ow[q] = arow[q];
+      for (int q = 0; q < KV; ++q) {
+        if constexpr (SPLIT) ow[q] = __builtin_bit_cast(float, bf_pair(arow[q]));
+        else ow[q] = arow[q];
+        lt[nn * LS + g * KV + q] = ow[q];
+      }
     }
     if constexpr (kPReg && !SPLIT) {
       fp.product(ow, acc);
@@ -1387,7 +1421,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
           if constexpr (kNatU) {
             mine[m * LS + 16 * t + nn] = v;
           } else if (rok[r] && stok[t]) {
-            if constexpr (kNat)
+            if constexpr (sizeof(R) == 4)
               __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v),
                                                     tile_rsrc(cslab, tile), (int)tvo[r], 64 * t, 0);
             else
@@ -1454,6 +1488,7 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   const int MT = S <= 16 ? 1 : (S <= 32 ? 2 : 4);
   const int threads = 2 * a.C * 64;
   const size_t lds = mfma_lds<R>(a.C, S, !post);
+  const bool nat = sizeof(R) == 4 && use_nat_rows(S, a.C);
   // LDS holds no codes of a chunk any more, and its rows are padded at 64 states; a chunk too large
   // for the codes stays refused
   const size_t codes = 2 * (size_t)a.tiles_per_chunk * kTile;
@@ -1468,21 +1503,28 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   HX_REQUIRE((size_t)(a.N + 16) * a.C * S + 64 < ((size_t)1 << 31), HX_ERR_UNSUPPORTED,
              "dense-state slab exceeds 31-bit offsets");
   dim3 grid(a.nchunks, a.K, width);
-#define HX_MF(KER, MTV, KVV, TV, RV)                                                         \
+#define HX_MF(KER, MTV, KVV, TV, RV, ...)                                                    \
   do {                                                                                       \
-    auto kern = KER<R, MTV, KVV, TV, RV, SPLIT>;                                             \
+    auto kern = KER<R, MTV, KVV, TV, RV, SPLIT, ##__VA_ARGS__>;                              \
     if (lds > 64 * 1024)                                                                     \
       HX_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                    \
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
     kern<<<grid, threads, lds, st>>>(a, nodes, S);                                           \
   } while (0)
-#define HX_MF_ALL(KER, MTV, KVV)                                                             \
+#define HX_MF_ALL(KER, MTV, KVV, ...)                                                        \
   if (tips == HX_TIPS_CODES) {                                                               \
-    if (root) HX_MF(KER, MTV, KVV, HX_TIPS_CODES, true);                                     \
-    else HX_MF(KER, MTV, KVV, HX_TIPS_CODES, false);                                         \
+    if (root) HX_MF(KER, MTV, KVV, HX_TIPS_CODES, true, ##__VA_ARGS__);                      \
+    else HX_MF(KER, MTV, KVV, HX_TIPS_CODES, false, ##__VA_ARGS__);                          \
   } else {                                                                                   \
-    if (root) HX_MF(KER, MTV, KVV, HX_TIPS_DENSE, true);                                     \
-    else HX_MF(KER, MTV, KVV, HX_TIPS_DENSE, false);                                         \
+    if (root) HX_MF(KER, MTV, KVV, HX_TIPS_DENSE, true, ##__VA_ARGS__);                      \
+    else HX_MF(KER, MTV, KVV, HX_TIPS_DENSE, false, ##__VA_ARGS__);                          \
+  }
+// NatRows or operands, for the kernels that have both
+#define HX_MF_NAT(MAC, ...)                                                                  \
+  if constexpr (sizeof(R) == 4) {                                                            \
+    if (nat) { MAC(__VA_ARGS__, true) } else { MAC(__VA_ARGS__, false) }                     \
+  } else {                                                                                   \
+    MAC(__VA_ARGS__, false)                                                                  \
   }
 // the root launch of the post-order (k_post_mfma_r serves every other level)
 #define HX_MF_ROOT(MTV, KVV)                                                                 \
@@ -1499,21 +1541,21 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
     PassArgs<R> b = a;
     b.tiles_per_chunk = post_level_tiles(a.ntiles, S, a.C, a.K, width, sizeof(R) == 8);
     grid.x = (a.ntiles + b.tiles_per_chunk - 1) / b.tiles_per_chunk;
-#define HX_MFR(MTV, KVV)                                                                     \
+#define HX_MFR(MTV, KVV, NATV)                                                               \
   if (tips == HX_TIPS_CODES)                                                                 \
-    k_post_mfma_r<R, MTV, KVV, HX_TIPS_CODES, SPLIT><<<grid, threads, lds_r, st>>>(b, nodes, \
-                                                                                   S);       \
+    k_post_mfma_r<R, MTV, KVV, HX_TIPS_CODES, SPLIT, NATV>                                   \
+        <<<grid, threads, lds_r, st>>>(b, nodes, S);                                         \
   else                                                                                       \
-    k_post_mfma_r<R, MTV, KVV, HX_TIPS_DENSE, SPLIT><<<grid, threads, lds_r, st>>>(b, nodes, \
-                                                                                   S);
+    k_post_mfma_r<R, MTV, KVV, HX_TIPS_DENSE, SPLIT, NATV>                                   \
+        <<<grid, threads, lds_r, st>>>(b, nodes, S);
     if (MT == 1) {
-      HX_MFR(1, 4)
+      HX_MF_NAT(HX_MFR, 1, 4)
     } else if (MT == 4) {
-      HX_MFR(4, 16)
+      HX_MFR(4, 16, sizeof(R) == 4)
     } else if (S <= 20) {
-      HX_MFR(2, 5)
+      HX_MF_NAT(HX_MFR, 2, 5)
     } else {
-      HX_MFR(2, 8)
+      HX_MFR(2, 8, sizeof(R) == 4)
     }
 #undef HX_MFR
   } else if (post) {
@@ -1525,12 +1567,13 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
       HX_MF_ROOT(4, 16)
     }
   } else if (MT == 1) {
-    HX_MF_ALL(k_pre_mfma_r, 1, 4)
+    HX_MF_NAT(HX_MF_ALL, k_pre_mfma_r, 1, 4)
   } else if (MT == 2) {
-    if (S <= 20) { HX_MF_ALL(k_pre_mfma_r, 2, 5) } else { HX_MF_ALL(k_pre_mfma_r, 2, 8) }
+    if (S <= 20) { HX_MF_NAT(HX_MF_ALL, k_pre_mfma_r, 2, 5) }
+    else { HX_MF_ALL(k_pre_mfma_r, 2, 8, sizeof(R) == 4) }
   } else if constexpr (sizeof(R) == 4) {
     HX_REQUIRE(a.ppad != nullptr, HX_ERR_INVALID_ARGUMENT, "padded P copies missing");
-    HX_MF_ALL(k_pre_mfma_r, 4, 16)
+    HX_MF_ALL(k_pre_mfma_r, 4, 16, true)
   } else {
     HX_MF_ALL(k_pre_mfma, 4, 16)
   }
