@@ -350,26 +350,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 //   m_h  = P_h L_h,  Ut_1 = U * m_2,  Ut_2 = U * m_1        (per category)
 //   lik  = sum_c p_c sum_s U m_1 m_2                         (scaled site likelihood)
 //   G_h[c][i][j] = sum over patterns of (w p_c / lik) Ut_h[c][i] L_h[c][j], or
-//   dtau_h[c]    = sum over patterns of (w p_c / lik) Ut_h[c] . (dP_h/dtau L_h)[c]
+//   dtau_h[c]    = sum over i, j of G_h[c][i][j] dP_h/dtau[c][i][j]
 //   U_h  = P_h^T Ut_h with one power-of-two rescale over all categories
 // Every term is a ratio, so the scales of U and L cancel. A dropped cherry's partial is rebuilt
 // from its two tips' codes; the continuing adjoint stays in registers, a pushed one too when
 // nothing else is pushed before its pop, and otherwise in the child's own partials row, which has
 // been read by then.
 //
-// All of an entry's loads are issued in the entry before it, after that entry's stores; an entry
-// with nothing to read issues nothing.
+// All of an entry's loads are issued in the entry before it, ahead of that entry's store (the
+// adjoint it pushes, which the next entry never pops); an empty range reads nothing.
 //
 // G: each wave writes Ut (rows 4c + i) and (w / lik) L (rows 4c + j) to LDS, pattern minor, and
 // reads them back as the operands of 16 v_mfma_f32_4x4x1_16b_f32, whose block 4c + q sums
 // category c's 4 x 4 outer products over patterns 16q .. 16q + 15; row rotations add the four
 // blocks q. The W waves' G meet in LDS one entry later (one barrier per entry, two buffers).
 //
-// dtau: the lane's own terms of both children and all categories are summed over eight lanes by
-// pairwise merges, which leave value (lane mod 8) in each lane, kept in LDS for kTauGroup
-// entries and then summed over lanes and waves in FP64: no transposes, and a barrier per group.
-constexpr int kXS = 68;        // row stride (floats) of the LDS pattern transposes
-constexpr int kTauGroup = 8;   // entries whose dtau terms meet at one barrier
+// dtau: the 16 sums of a (child, category) meet dP/dtau in FP64 on their way out. Rows of dP/dtau sum
+// to zero, so this contraction cancels. Done in FP32, per pattern and ahead of the sums, it needs no
+// transposes, but its error against 64 bits was 1.04 to 1.1 times as large (the calls 60 taxa x 431
+// patterns and 413 x 9871 at 8 samples took 135 and 1380 us so, 164 and 1504 as here); in FP64 per
+// pattern they took 177 and 1854.
+constexpr int kXS = 68;  // row stride (floats) of the LDS pattern transposes
 
 // v + (v from the lane `ROT` below in the same row of 16 lanes, cyclically): DPP row_ror
 template <int ROT>
@@ -378,23 +379,7 @@ __device__ __forceinline__ float add_row_ror(float v) {
   return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v),
                                                                  0x120 + ROT, 0xF, 0xF, true));
 }
-// v moved between lanes by a DPP control word that reaches every lane
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-  return __builtin_bit_cast(
-      float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
-}
-// One merge step of two lane sums: lanes with `odd` end with b's partial sums, the others with
-// a's, each over the lane and its partner under CTRL (which flips `odd`).
-template <int CTRL>
-__device__ __forceinline__ float merge(float a, float b, bool odd) {
-  return (odd ? b : a) + dpp<CTRL>(odd ? a : b);
-}
-constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kHalfMirror = 0x141;  // quad_perm, quad_perm, row_half_mirror
-
-constexpr size_t pre4_lds_floats(bool tau) {
-  return tau ? 2 * kTauGroup * kPreWalkW * 64 : (size_t)kPreWalkW * 3 * 16 * kXS + 4 * kPreWalkW * 64;
-}
+constexpr size_t kPre4LdsFloats = (size_t)kPreWalkW * 3 * 16 * kXS + 4 * kPreWalkW * 64;
 
 template <int TIPS, int CM, bool EXACT, bool TAU>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CM == 4 ? 2 : 3))) void
@@ -414,11 +399,9 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
   float* sm = reinterpret_cast<float*>(smem_raw);
   float* xs = sm + (size_t)wave * 3 * 16 * kXS;  // rows 4c + i: (w / lik) Ut[c][i] of one child
   float* ls = xs + 16 * kXS;                     // [2] rows 4c + j: L[c][j] (a tip: rows j)
-  float* red = TAU ? sm : sm + (size_t)W * 3 * 16 * kXS;  // [2][2][W][64]; TAU [2][group][W][64]
-  int* ids = reinterpret_cast<int*>(sm + pre4_lds_floats(TAU));  // TAU: [2][group][2] branches
-  f4* tbl = reinterpret_cast<f4*>(ids + (TAU ? 4 * kTauGroup : 0));
-  if constexpr (!TAU)
-    for (int i = lane; i < 3 * 16 * kXS; i += 64) xs[i] = 0.f;  // rows of absent categories
+  float* red = sm + (size_t)W * 3 * 16 * kXS;    // [2][2][W][64]
+  f4* tbl = reinterpret_cast<f4*>(sm + kPre4LdsFloats);
+  for (int i = lane; i < 3 * 16 * kXS; i += 64) xs[i] = 0.f;  // rows of absent categories
   stage_table<TIPS>(a, tbl);
 
   const float w = val ? (float)a.weights[n] : 0.f;
@@ -469,9 +452,10 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
   };
 
   struct Small {
-    float p[2], pt[2], dp[2], g[2][2];  // P, P^T, dP/dtau; P of a dropped cherry's tips
+    float p[2], pt[2], g[2][2];         // P, P^T; P of a dropped cherry's tips
     int code[2][2];                     // a tip's code, or a dropped cherry's two
     f4 t[2];                            // dense tips
+    float dp;                           // TAU: this thread's value of dP/dtau (flush_g)
   };
   Small in[2];
   f4 U[CM], held[CM], L0[CM], L1[CM], Up[CM];
@@ -489,12 +473,13 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
   auto Lh = [&](auto h) -> f4(&)[CM] {
     if constexpr (decltype(h)::value == 0) return L0; else return L1;
   };
+  // the statistic of thread t: value t mod CS of child t / CS's G
+  const int CS = C * 16, sh = (int)threadIdx.x >= CS, se = threadIdx.x % CS;
   auto fetch_small = [&](const Entry& e, Small& x) {
     each<2>([&](auto hc) {
       constexpr int h = decltype(hc)::value;
       const int ch = h ? e.c2 : e.c1;
       x.p[h] = buf_load(pbuf, pf, ch * C * 64);
-      if constexpr (TAU) x.dp[h] = buf_load(dbuf, pf, ch * C * 64);
       const int kd = kind(e.m, h);
       if constexpr (TIPS == HX_TIPS_CODES) {
         x.code[h][0] = tip_code(cbuf, kd == 0 ? ch : e.g[2 * h], a.N, nc);
@@ -506,6 +491,7 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
       }
       x.pt[h] = buf_load(pbuf, pt, ch * C * 64);
     });
+    if constexpr (TAU) x.dp = buf_load(dbuf, 4u * ((sh ? e.c2 : e.c1) * CS + se), 0);
   };
   auto fetch_rows = [&](const Entry& e) {
     load_rows(e.c1, kind(e.m, 0) == 2, L0, std::true_type{});
@@ -513,42 +499,25 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
     load_rows(e.p, (e.m & 3) == 2, Up, std::false_type{});
   };
 
-  // the statistics of entry i meet in LDS during entry i + 1 (G) or its group (dtau)
-  const int CS = C * 16;
-  float spc = 0.f;
-  if constexpr (!TAU) spc = a.props[(size_t)k * a.props_ks + ((threadIdx.x % CS) >> 4)];
-  auto flush_g = [&](int b1, int b2, int par) {
+  // the statistics of entry i meet in LDS during entry i + 1
+  const float spc = a.props[(size_t)k * a.props_ks + (se >> 4)];
+  auto flush_g = [&](int b1, int b2, float dp, int par) {
     lds_barrier();
     if ((int)threadIdx.x < 2 * CS) {
-      const int h = (int)threadIdx.x >= CS, se = threadIdx.x - h * CS;
       float s = 0.f;
 #pragma unroll
-      for (int q = 0; q < W; ++q) s += red[((par * 2 + h) * W + q) * 64 + se];
-      a.gpart[(((size_t)(h ? b2 : b1) * a.K + k) * a.nchunks + chunk) * CS + se] = s * spc;
-    }
-  };
-  // group gi's sums: thread (entry, value, wave), over the wave's 64 / NV partial sums
-  constexpr int NV = 2 * CM;
-  auto flush_tau = [&](int gi, int cnt) {
-    lds_barrier();
-    const int par = gi & 1;
-    const int e = threadIdx.x / (4 * NV), v = (threadIdx.x >> 2) % NV, part = threadIdx.x & 3;
-    double s = 0.0;
-    if (e < cnt) {
-      const float* src = red + ((size_t)(par * kTauGroup + e) * W + part) * 64 + v;
+      for (int q = 0; q < W; ++q) s += red[((par * 2 + sh) * W + q) * 64 + se];
+      const size_t at = ((size_t)(sh ? b2 : b1) * a.K + k) * a.nchunks + chunk;
+      if constexpr (TAU) {
+        double t = (double)(s * spc) * (double)dp;
 #pragma unroll
-      for (int q = 0; q < 64 / NV; ++q) s += (double)src[q * NV];
-    }
-    s += __shfl_xor(s, 1);
-    s += __shfl_xor(s, 2);
-    const int h = v / CM, c = v % CM;
-    if (e < cnt && part == 0 && c < C) {
-      const int b = ids[(par * kTauGroup + e) * 2 + h];
-      a.gtau[(((size_t)b * a.K + k) * a.nchunks + chunk) * C + c] =
-          s * (double)a.props[(size_t)k * a.props_ks + c];
+        for (int o = 1; o < 16; o <<= 1) t += __shfl_xor(t, o);
+        if ((se & 15) == 0) a.gtau[at * C + (se >> 4)] = t;
+      } else {
+        a.gpart[at * CS + se] = s * spc;
+      }
     }
   };
-  static_assert(4 * NV * kTauGroup <= 256 && W == 4, "a thread per (entry, value, wave) of a group");
 
   Entry cur = entry(0);
   __builtin_amdgcn_sched_barrier(0);
@@ -557,6 +526,7 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
   fetch_rows(cur);
   __builtin_amdgcn_sched_barrier(0);
   int fb1 = 0, fb2 = 0;
+  float fdp = 0.f;
   auto step = [&](int i, auto slot) __attribute__((always_inline)) {
     constexpr int sl = decltype(slot)::value;
     using H0 = std::integral_constant<int, 0>;
@@ -576,8 +546,8 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
 #pragma unroll
       for (int c = 0; c < CM; ++c) U[c] = held[c];
     }
-    // m_h = P_h L_h; without TAU, L_h's rows go to LDS for the statistic
-    f4 m[2][CM], tv[2];
+    // m_h = P_h L_h; L_h's rows go to LDS for the statistic
+    f4 m[2][CM];
     each<2>([&](auto hc) {
       constexpr int h = decltype(hc)::value;
       f4(&L)[CM] = Lh(hc);
@@ -587,12 +557,8 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
         if constexpr (TIPS == HX_TIPS_CODES) t = tbl[x.code[h][0]];
         else t = x.t[h];
         mv4<CM>(x.p[h], [&](auto) { return t; }, m[h]);
-        if constexpr (TAU) {
-          tv[h] = t;
-        } else {
 #pragma unroll
-          for (int s = 0; s < 4; ++s) ls[(16 * h + s) * kXS + lane] = t[s];
-        }
+        for (int s = 0; s < 4; ++s) ls[(16 * h + s) * kXS + lane] = t[s];
       } else {
         if constexpr (TIPS == HX_TIPS_CODES) {
           if (kd == 1) {
@@ -606,18 +572,15 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
           }
         }
         mv4<CM>(x.p[h], [&](auto c) { return L[c]; }, m[h]);
-        if constexpr (!TAU) {
 #pragma unroll
-          for (int c = 0; c < CM; ++c)
-            if (EXACT || c < C)
+        for (int c = 0; c < CM; ++c)
+          if (EXACT || c < C)
 #pragma unroll
-              for (int s = 0; s < 4; ++s) ls[(16 * h + 4 * c + s) * kXS + lane] = L[c][s];
-        }
+            for (int s = 0; s < 4; ++s) ls[(16 * h + 4 * c + s) * kXS + lane] = L[c][s];
       }
       __builtin_amdgcn_sched_barrier(0);  // one child's registers at a time
     });
-    // (!TAU) the partials are used up: the next entry's
-    if constexpr (!TAU) fetch_rows(nxt);
+    fetch_rows(nxt);  // the partials are used up: the next entry's
     // Ut, in m's place: m[0] becomes Ut_2, m[1] becomes Ut_1
     float lik = 0.f;
 #pragma unroll
@@ -674,54 +637,14 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
         for (int r = 0; r < 4; ++r) dst[4 * r] = g[r];
       }
     };
-    if constexpr (!TAU) {
-      stat_rows(H0{});
-      // the barrier in here also keeps this entry's writes behind every read of entry i - 2
-      if (i > 0) flush_g(fb1, fb2, (i - 1) & 1);
-      fb1 = cur.c1;
-      fb2 = cur.c2;
-      stat_put(0, stat_mfma(0));
-      stat_rows(H1{});
-    } else {
-      float v[NV];
-      each<2>([&](auto hc) {
-        constexpr int h = decltype(hc)::value;
-        f4 z[CM];  // dP_h L_h
-        if (kind(m_, h) == 0) mv4<CM>(x.dp[h], [&](auto) { return tv[h]; }, z);
-        else mv4<CM>(x.dp[h], [&](auto c) { return Lh(hc)[c]; }, z);
-#pragma unroll
-        for (int c = 0; c < CM; ++c) {
-          float t = 0.f;
-          if (EXACT || c < C)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) t = fmaf(Ut(hc)[c][s], z[c][s], t);
-          v[h * CM + c] = coef * t;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      });
-      fetch_rows(nxt);  // the partials are used up: the next entry's
-      // value j ends in the lanes congruent to j modulo NV
-      float r;
-      const bool o1 = lane & 1, o2 = lane & 2, o4 = lane & 4;
-      if constexpr (NV == 2) {
-        r = merge<kXor1>(v[0], v[1], o1);
-      } else if constexpr (NV == 4) {
-        r = merge<kXor2>(merge<kXor1>(v[0], v[1], o1), merge<kXor1>(v[2], v[3], o1), o2);
-      } else {
-        // the half-row mirror flips the lane's three low bits: where bit 2 is set, values 0-3 are
-        // laid out in reverse, and where it is clear values 4-7 are, so that partners match
-        const bool s1 = o1 != o4, s2 = o2 != o4;
-        const float a0 = merge<kXor2>(merge<kXor1>(v[0], v[1], s1), merge<kXor1>(v[2], v[3], s1), s2);
-        const float a1 =
-            merge<kXor2>(merge<kXor1>(v[4], v[5], !s1), merge<kXor1>(v[6], v[7], !s1), !s2);
-        r = merge<kHalfMirror>(a0, a1, o4);
-      }
-      const int gi = i / kTauGroup, ge = i % kTauGroup, par = gi & 1;
-      // the barrier in here also keeps this group's writes behind every read of group gi - 2
-      if (ge == 0 && i > 0) flush_tau(gi - 1, kTauGroup);
-      red[((size_t)(par * kTauGroup + ge) * W + wave) * 64 + lane] = r;
-      if (wave == 0 && lane < 2) ids[(par * kTauGroup + ge) * 2 + lane] = lane ? cur.c2 : cur.c1;
-    }
+    stat_rows(H0{});
+    // the barrier in here also keeps this entry's writes behind every read of entry i - 2
+    if (i > 0) flush_g(fb1, fb2, fdp, (i - 1) & 1);
+    fb1 = cur.c1;
+    fb2 = cur.c2;
+    if constexpr (TAU) fdp = x.dp;
+    stat_put(0, stat_mfma(0));
+    stat_rows(H1{});
 
     __builtin_amdgcn_sched_barrier(0);
     // adjoints of internal children
@@ -743,7 +666,7 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
       mv4<CM>(x.pt[1], [&](auto c) { return Ut(H1{})[c]; }, U);
       rescale<CM, EXACT>(U, C);
     }
-    if constexpr (!TAU) stat_put(1, stat_mfma(1));
+    stat_put(1, stat_mfma(1));
     cur = nxt;
   };
   for (int i = 0; i < nprog; ++i) {
@@ -751,12 +674,7 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
     if (++i == nprog) break;
     step(i, std::integral_constant<int, 1>{});
   }
-  if constexpr (TAU) {
-    const int gi = (nprog - 1) / kTauGroup;
-    flush_tau(gi, nprog - gi * kTauGroup);
-  } else {
-    flush_g(fb1, fb2, (nprog - 1) & 1);
-  }
+  flush_g(fb1, fb2, fdp, (nprog - 1) & 1);
 }
 
 // -------------------------------------------------------------------- launchers
@@ -805,8 +723,7 @@ int launch_pre_walk4(const PassArgs<float>& a, const int32_t* prog, int nprog, i
   HX_REQUIRE(a.C >= 1 && a.C <= kPreWalkMaxC && a.nchunks == (a.ntiles + kPreWalkW - 1) / kPreWalkW,
              HX_ERR_UNSUPPORTED, "pre-order walk: chunking does not match the workgroup's tiles");
   const bool tau = a.mats_dt != nullptr;
-  const size_t lds = pre4_lds_floats(tau) * 4 + (tau ? 4 * kTauGroup * 4 : 0) +
-                     table_bytes(tips, a.ncodes);
+  const size_t lds = kPre4LdsFloats * 4 + table_bytes(tips, a.ncodes);
   HX_REQUIRE(lds <= 64 * 1024, HX_ERR_UNSUPPORTED, "pre-order walk: LDS");
   const auto kern = a.C == 1   ? pre_kernel<1, true>(tips, tau)
                     : a.C == 2 ? pre_kernel<2, true>(tips, tau)
