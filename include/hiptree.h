@@ -121,6 +121,17 @@ int hx_loglik(hx_plan_t plan, int S, int N, int C, int K, int dtype,
               double* out_loglik, double* out_dfreqs, double* out_dprops,
               hx_stream_t stream);
 
+/* hx_loglik for a value that no gradient follows (same arguments, same results): the
+ * partials need not be kept, so what is left in the workspace is of no use. */
+int hx_loglik_value(hx_plan_t plan, int S, int N, int C, int K, int dtype,
+                    int tip_kind, const void* tips, const void* tip_table, int ncodes,
+                    const double* weights, const void* mats,
+                    const void* freqs, int freqs_batched,
+                    const void* props, int props_batched,
+                    void* workspace, size_t workspace_bytes,
+                    double* out_loglik, double* out_dfreqs, double* out_dprops,
+                    hx_stream_t stream);
+
 /* Pre-order adjoint over the partials left in `workspace` by hx_loglik
  * (consumed: the partials are overwritten in place). Output:
  *   out_dmats [K][B][C][S][S] double = d loglik / d mats. */

@@ -11,9 +11,9 @@ pytestmark = pytest.mark.gpu
 F64 = torch.float64
 
 
-def _call(gpu, post, tips, table, weights, mats, mats_dt, dtype):
+def _call(gpu, post, tips, table, weights, mats, mats_dt, dtype, first=2):
     """(logL [K], d/dtau [K, B, C]) of hx_loglik and hx_loglik_grad_tau; tips [T, N] codes with a
-    table, or [T, N, S]."""
+    table, or [T, N, S]. first: the gradient mode whose workspace size hx_loglik is told."""
     from torchtree_amd import _lib
     from torchtree_amd.likelihood import Plan, _dtype_code
 
@@ -36,7 +36,8 @@ def _call(gpu, post, tips, table, weights, mats, mats_dt, dtype):
             0 if dense else table.shape[0], weights.data_ptr(), mats.data_ptr())
     tail = (freqs.data_ptr(), 0, props.data_ptr(), 0, ws.data_ptr(), nb)
     st = _lib.stream_handle(gpu)
-    _lib.check(lib.hx_loglik(*head, *tail, ll.data_ptr(), 0, 0, st))
+    small = plan.workspace_bytes(S, N, C, K, code, first)
+    _lib.check(lib.hx_loglik(*head, *tail[:-1], small, ll.data_ptr(), 0, 0, st))
     _lib.check(lib.hx_loglik_grad_tau(*head, mats_dt.data_ptr(), *tail, dt.data_ptr(), st))
     torch.cuda.synchronize()
     return ll.cpu(), dt.cpu()
@@ -105,3 +106,22 @@ def test_grad_tau_contracts_in_64_bits(gpu, C):
     tips = slice(0, T)  # branches of tips, whose partials are ones exactly
     assert torch.allclose(ref[:, tips].sum(-1), weights.sum().expand(K, T), rtol=1e-5)
     assert float((dt[:, tips] - ref[:, tips]).abs().max() / ref[:, tips].abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, F64])
+@pytest.mark.parametrize("shape,T,N,C,S", [("balanced", 16, 64, 4, 4), ("caterpillar", 20, 33, 4, 20)])
+def test_partials_are_kept_whatever_size_is_told(gpu, shape, T, N, C, S, dtype):
+    """A caller with one buffer for both calls may tell hx_loglik the size without a gradient: its
+    partials are there all the same."""
+    from torchtree_amd import _lib
+
+    rng = np.random.default_rng(T)
+    post, K, B = _tree(shape, T), 2, 2 * T - 2
+    mats = torch.tensor(rng.uniform(0.1, 1.0, (K, B, C, S, S)) + S * np.eye(S))
+    mats = mats / mats.sum(-1, keepdim=True)
+    mats_dt = torch.tensor(rng.standard_normal((K, B, C, S, S)))
+    weights = torch.ones(N, dtype=F64)
+    args = (post, torch.tensor(rng.integers(0, S, (T, N))), torch.eye(S), weights, mats, mats_dt, dtype)
+    told = _call(gpu, *args, first=_lib.HX_GRAD_NONE)
+    for a, b in zip(told, _call(gpu, *args)):
+        assert torch.equal(a, b)

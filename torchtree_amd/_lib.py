@@ -42,6 +42,10 @@ _SIGNATURES = {
                            _c_int, _vp, _vp, _c_int,
                            _dp, _vp, _vp, _c_int, _vp, _c_int,
                            _vp, _c_size, _dp, _dp, _dp, _vp]),
+    "hx_loglik_value": (_c_int, [_vp, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                 _c_int, _vp, _vp, _c_int,
+                                 _dp, _vp, _vp, _c_int, _vp, _c_int,
+                                 _vp, _c_size, _dp, _dp, _dp, _vp]),
     "hx_loglik_grad_mats": (_c_int, [_vp, _c_int, _c_int, _c_int, _c_int, _c_int,
                                      _c_int, _vp, _vp, _c_int,
                                      _dp, _vp, _vp, _c_int, _vp, _c_int,

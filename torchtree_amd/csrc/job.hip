@@ -320,10 +320,10 @@ static int job_eval_in(hx_job_t job, int K, const double* bls, double* out_logli
   if (grad) hx::fill0(dt_acc, nt, st);
   for (int s = 0; s < job->nslices; ++s) {
     const int n = job->slice_n[s];
-    rc = hx_loglik(job->plan, job->S, n, job->C, K, job->dtype, HX_TIPS_CODES, job->d_codes[s],
-                   job->d_table, job->ncodes, job->d_weights[s], mats, job->d_freqs, 0,
-                   job->d_props, 0, base + w.prune, w.prune_bytes, ll_tmp, nullptr, nullptr,
-                   stream);
+    rc = (grad ? hx_loglik : hx_loglik_value)(
+        job->plan, job->S, n, job->C, K, job->dtype, HX_TIPS_CODES, job->d_codes[s], job->d_table,
+        job->ncodes, job->d_weights[s], mats, job->d_freqs, 0, job->d_props, 0, base + w.prune,
+        w.prune_bytes, ll_tmp, nullptr, nullptr, stream);
     if (rc != HX_OK) return rc;
     hx::accum(out_loglik, ll_tmp, K, st);
     if (grad) {

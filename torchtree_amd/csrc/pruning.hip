@@ -198,6 +198,7 @@ struct CallArgs {
   size_t ws_bytes;
   int grad_mode;
   const void* mats_dt;
+  bool value_only;  // hx_loglik_value: no gradient follows
 };
 
 static int validate(const CallArgs& c) {
@@ -293,10 +294,8 @@ static int run_post(const CallArgs& c, double* out_l, double* out_f, double* out
   const PassArgs<R> a = make_args<R>(c);
   const hx_plan_s* plan = c.plan;
   int nparts = a.nchunks;
-  // no gradient can follow in a workspace that has no room for one (each gradient call checks for
-  // its own): then the walks need not keep the partials
-  const bool store = c.ws_bytes >= std::min(ws_layout(plan, c.S, c.N, c.C, c.K, c.dtype, 1).total,
-                                            ws_layout(plan, c.S, c.N, c.C, c.K, c.dtype, 2).total);
+  // without a gradient to follow the walks need not keep the partials
+  const bool store = !c.value_only;
   bool dwalk = false;
   if constexpr (std::is_same<R, float>::value) {
     if (runs_dwalk(c)) {
@@ -414,6 +413,15 @@ static int run_pre(const CallArgs& c, double* out, hipStream_t st) {
   return HX_OK;
 }
 
+static int loglik(const CallArgs& c, double* out_l, double* out_f, double* out_p, hx_stream_t stream) {
+  const int rc = validate(c);
+  if (rc != HX_OK) return rc;
+  HX_REQUIRE(out_l != nullptr, HX_ERR_INVALID_ARGUMENT, "null output");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  return c.dtype == HX_F64 ? run_post<double>(c, out_l, out_f, out_p, st)
+                           : run_post<float>(c, out_l, out_f, out_p, st);
+}
+
 }  // namespace hx
 
 extern "C" {
@@ -442,14 +450,19 @@ int hx_loglik(hx_plan_t plan, int S, int N, int C, int K, int dtype, int tip_kin
               const void* freqs, int freqs_batched, const void* props, int props_batched,
               void* workspace, size_t workspace_bytes, double* out_loglik, double* out_dfreqs,
               double* out_dprops, hx_stream_t stream) {
-  hx::CallArgs c{plan, S, N, C, K, dtype, tip_kind, tips, tip_table, ncodes, weights, mats,
-                 freqs, freqs_batched, props, props_batched, workspace, workspace_bytes, 0, nullptr};
-  int rc = hx::validate(c);
-  if (rc != HX_OK) return rc;
-  HX_REQUIRE(out_loglik != nullptr, HX_ERR_INVALID_ARGUMENT, "null output");
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (dtype == HX_F64) return hx::run_post<double>(c, out_loglik, out_dfreqs, out_dprops, st);
-  return hx::run_post<float>(c, out_loglik, out_dfreqs, out_dprops, st);
+  return hx::loglik({plan, S, N, C, K, dtype, tip_kind, tips, tip_table, ncodes, weights, mats, freqs,
+                     freqs_batched, props, props_batched, workspace, workspace_bytes, 0, nullptr, false},
+                    out_loglik, out_dfreqs, out_dprops, stream);
+}
+
+int hx_loglik_value(hx_plan_t plan, int S, int N, int C, int K, int dtype, int tip_kind,
+                    const void* tips, const void* tip_table, int ncodes, const double* weights,
+                    const void* mats, const void* freqs, int freqs_batched, const void* props,
+                    int props_batched, void* workspace, size_t workspace_bytes, double* out_loglik,
+                    double* out_dfreqs, double* out_dprops, hx_stream_t stream) {
+  return hx::loglik({plan, S, N, C, K, dtype, tip_kind, tips, tip_table, ncodes, weights, mats, freqs,
+                     freqs_batched, props, props_batched, workspace, workspace_bytes, 0, nullptr, true},
+                    out_loglik, out_dfreqs, out_dprops, stream);
 }
 
 int hx_loglik_grad_mats(hx_plan_t plan, int S, int N, int C, int K, int dtype, int tip_kind,
@@ -458,7 +471,7 @@ int hx_loglik_grad_mats(hx_plan_t plan, int S, int N, int C, int K, int dtype, i
                         int props_batched, void* workspace, size_t workspace_bytes,
                         double* out_dmats, hx_stream_t stream) {
   hx::CallArgs c{plan, S, N, C, K, dtype, tip_kind, tips, tip_table, ncodes, weights, mats,
-                 freqs, freqs_batched, props, props_batched, workspace, workspace_bytes, 1, nullptr};
+                 freqs, freqs_batched, props, props_batched, workspace, workspace_bytes, 1, nullptr, false};
   int rc = hx::validate(c);
   if (rc != HX_OK) return rc;
   HX_REQUIRE(out_dmats != nullptr, HX_ERR_INVALID_ARGUMENT, "null output");
@@ -474,7 +487,7 @@ int hx_loglik_grad_tau(hx_plan_t plan, int S, int N, int C, int K, int dtype, in
                        size_t workspace_bytes, double* out_dtau, hx_stream_t stream) {
   hx::CallArgs c{plan, S, N, C, K, dtype, tip_kind, tips, tip_table, ncodes, weights, mats,
                  freqs, freqs_batched, props, props_batched, workspace, workspace_bytes, 2,
-                 mats_dtau};
+                 mats_dtau, false};
   int rc = hx::validate(c);
   if (rc != HX_OK) return rc;
   HX_REQUIRE(out_dtau != nullptr && mats_dtau != nullptr, HX_ERR_INVALID_ARGUMENT,

@@ -261,7 +261,7 @@ class Pruning:
         dfreqs = torch.empty(K, S, dtype=torch.float64, device=dev) if want_root_grads else None
         dprops = torch.empty(K, C, dtype=torch.float64, device=dev) if want_root_grads else None
         with timing.phase("postorder", self._launches(_lib.HX_GRAD_NONE, S, C, code, K)):
-            rc = lib.hx_loglik(
+            rc = (lib.hx_loglik if want_root_grads else lib.hx_loglik_value)(
             self.plan.handle, S, self.N, C, K, code, self.tips.kind,
             _lib.ptr(tips_p), _lib.ptr(table_p), self.tips.ncodes,
             _lib.ptr(self.weights), _lib.ptr(mats),
