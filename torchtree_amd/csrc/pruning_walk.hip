@@ -563,12 +563,14 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
         if constexpr (TIPS == HX_TIPS_CODES) {
           if (kd == 1) {
             // the cherry's partial before the post-order walk's power-of-two rescale: every
-            // term below is a ratio in it
+            // term below is a ratio in it. Of two such children one is rescaled, since the
+            // product of two small ones could underflow.
             const f4 t0 = tbl[x.code[h][0]], t1 = tbl[x.code[h][1]];
             mv4<CM>(x.g[h][0], [&](auto) { return t0; }, L);
             mv4<CM>(x.g[h][1], [&](auto) { return t1; }, m[h]);
 #pragma unroll
             for (int c = 0; c < CM; ++c) L[c] *= m[h][c];
+            if (h == 0 && kind(m_, 1) == 1) rescale<CM, EXACT>(L, C);
           }
         }
         mv4<CM>(x.p[h], [&](auto c) { return L[c]; }, m[h]);
