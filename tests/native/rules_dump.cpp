@@ -1,5 +1,6 @@
 // Dispatch rules of csrc/layout.hpp, for tests/test_rules.py: one query per input line.
 //   tiles S ntiles C K width f64    -> post_level_tiles
+//   tau ntiles C tiles_per_chunk    -> tau_chunk_tiles
 //   dwalk S C I levels ntiles K     -> use_dwalk
 #include <cstdio>
 #include <cstring>
@@ -13,6 +14,10 @@ int main() {
       int S, nt, C, K, w, f;
       if (std::scanf("%d %d %d %d %d %d", &S, &nt, &C, &K, &w, &f) != 6) return 1;
       std::printf("%d\n", hx::post_level_tiles(nt, S, C, K, w, f != 0));
+    } else if (!std::strcmp(what, "tau")) {
+      int nt, C, t;
+      if (std::scanf("%d %d %d", &nt, &C, &t) != 3) return 1;
+      std::printf("%d\n", hx::tau_chunk_tiles(nt, C, t));
     } else if (!std::strcmp(what, "dwalk")) {
       int S, C, I, h, nt, K;
       if (std::scanf("%d %d %d %d %d %d", &S, &C, &I, &h, &nt, &K) != 6) return 1;

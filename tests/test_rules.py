@@ -53,3 +53,11 @@ def test_dense_walk_only_where_its_chain_is_hidden(ask, S, C):
     on a bushy tree go by level, a caterpillar walks; past 32 states there is no walk."""
     assert ask([("dwalk", S, C, 127, 7, 1, 1), ("dwalk", S, C, 349, 18, 4, 1),
                 ("dwalk", S, C, 199, 199, 1, 1), ("dwalk", 33, C, 199, 199, 1, 1)]) == [0, 0, 1, 0]
+
+
+def test_tau_chunks_grow_with_the_patterns(ask):
+    """Short chunks where there are few blocks, longer ones before their set-ups outweigh that, never
+    longer than the d/dP chunks'."""
+    assert ask([("tau", 77, 4, 9), ("tau", 188, 4, 9), ("tau", 500, 4, 9), ("tau", 1000, 4, 8),
+                ("tau", 5000, 1, 40), ("tau", 188, 1, 9), ("tau", 500, 1, 9), ("tau", 7, 4, 7),
+                ("tau", 1, 1, 1)]) == [5, 6, 8, 8, 40, 5, 6, 5, 1]

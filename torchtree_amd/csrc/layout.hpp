@@ -182,6 +182,21 @@ inline bool use_dwalk(int S, int C, int I, int levels, int ntiles, int K) {
   return 8 + I * (a + b * C * past) <= levels * launch + I * blocks * C * v;
 }
 
+// Tiles per chunk of FP32 d/dtau at 33..64 states. A block's result is C doubles, so its chunk need not
+// be as long as a d/dP one's (9 or 10 tiles here), and shorter ones fill the levels' last rounds
+// better; but each sets P up, which weighs more the more blocks there are, and the sums may not depend
+// on the batch, so it is chosen from the patterns and the waves of a block (2 C). Whole calls of 20 to 150
+// taxa at 40 and 61 states against the d/dP chunks, one sample and 2 to 16: with 4 categories up to
+// 1217 patterns 5 tiles took 0.61 to 0.92 and 0.64 to 1.02, at 1600 to 3000 6 tiles 0.76 to 0.98 and
+// 0.80 to 1.04, at 4000 to 10000 8 tiles 0.92 to 1.00 and 0.94 to 1.01, where 5 lost up to 16 %; with
+// one category 5 tiles at 3000 0.69 to 0.76 and 0.81 to 1.02, 6 at 8000 0.81 to 0.92 and 0.89 to 1.03.
+// Past 16000 the d/dP chunks are 8 and more of themselves.
+inline int tau_chunk_tiles(int ntiles, int C, int tiles_per_chunk) {
+  const int x = ntiles * C;
+  const int t = ntiles > 1000 ? tiles_per_chunk : (x <= 320 ? 5 : (x <= 800 ? 6 : (x <= 2560 ? 8 : tiles_per_chunk)));
+  return t < tiles_per_chunk ? t : tiles_per_chunk;
+}
+
 // FP32 gradients at 33..64 states read P and P^T from zero-padded 64 x 64 copies.
 inline bool use_ppad(int S, int dtype, int grad_mode) {
   return grad_mode != 0 && dtype != HX_F64 && S > 32 && S <= 64;

@@ -361,16 +361,11 @@ template <typename R>
 static int run_pre(const CallArgs& c, double* out, hipStream_t st) {
   PassArgs<R> a = make_args<R>(c);
   const hx_plan_s* plan = c.plan;
-  // FP32 d/dtau at 33 to 64 states: a block's result is C doubles, so its chunk need not be as long
-  // as a d/dP one's, and shorter ones fill the levels' last rounds better (97 taxa x 1217 patterns
-  // at 8 samples, the whole call: 9 tiles 4712 us, 8: 4663, 6: 4559, 5: 4498, 4: 4721, 3: 4961,
-  // where each block's set-up weighs more). Past 1280 tiles (20000 patterns) there are blocks
-  // enough. The sums go where the post-order kept its exponents, which nothing reads any more: I K
-  // N 4 bytes for 2 I K nchunks C 8.
-  if (std::is_same<R, float>::value && c.grad_mode == 2 && use_mfma(c.C, c.S, c.dtype) &&
-      c.S > 32 && a.ntiles <= 1280) {
-    const int tpc = std::min(a.tiles_per_chunk, 5), nch = (a.ntiles + tpc - 1) / tpc;
-    if ((size_t)nch * c.C * 4 <= (size_t)c.N) {
+  // FP32 d/dtau at 33 to 64 states in shorter chunks (tau_chunk_tiles). The sums go where the
+  // post-order kept its exponents, which nothing reads any more: I K N 4 bytes for 2 I K nchunks C 8.
+  if (std::is_same<R, float>::value && c.grad_mode == 2 && use_mfma(c.C, c.S, c.dtype) && c.S > 32) {
+    const int tpc = tau_chunk_tiles(a.ntiles, c.C, a.tiles_per_chunk), nch = (a.ntiles + tpc - 1) / tpc;
+    if (tpc < a.tiles_per_chunk && (size_t)nch * c.C * 4 <= (size_t)c.N) {
       a.tiles_per_chunk = tpc;
       a.nchunks = nch;
       a.gtau = reinterpret_cast<double*>(a.scales);
