@@ -179,6 +179,14 @@ __device__ __forceinline__ void acc_outer(R (&g)[16], R w, const V4<R>& u, const
 // node's stores so the wait for it does not wait for them, and its exponent
 // comes from the lane's LDS stack. grid = (ntiles, ceil(K / W)), block = 64 W.
 // CM: categories rounded up to a power of two (EXACT: C == CM).
+__device__ __forceinline__ void store_row_f32(const __amdgpu_buffer_rsrc_t& r, unsigned off,
+                                              const V4<float>& v) {
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  const u4 w = {__float_as_uint(v.x[0]), __float_as_uint(v.x[1]), __float_as_uint(v.x[2]),
+                __float_as_uint(v.x[3])};
+  __builtin_amdgcn_raw_buffer_store_b128(w, r, (int)off, 0, 0);
+}
+
 template <typename R, int TIPS, int CM, bool EXACT>
 __global__ __launch_bounds__(CM >= 8 ? 256 : 1024) void k_post_walk(PassArgs<R> a, const R* __restrict__ mats,
                                                     const int4* __restrict__ prog, int nprog,
@@ -315,10 +323,21 @@ __global__ __launch_bounds__(CM >= 8 ? 256 : 1024) void k_post_walk(PassArgs<R> 
     if (last) break;
     // the next entry's stacked child, before this node's stores
     readback(stacked_of(f0, f1), xs);
-    R* p = base + (size_t)(v - a.T) * sstride;
+    if constexpr (sizeof(R) == 4) {
+      // this node's C rows of this sample as one raw buffer: no address on the vector units (2 % of
+      // the walk at 6 categories)
+      const R* node = a.partials + (size_t)(v - a.T) * sstride + (size_t)k * C * cstride;
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<R*>(node), (short)0, (int)((size_t)C * cstride * sizeof(R)), 0x00020000);
 #pragma unroll
-    for (int c = 0; c < CM; ++c)
-      if (EXACT || c < C) st4(p + (size_t)c * cstride, y[c]);
+      for (int c = 0; c < CM; ++c)
+        if (EXACT || c < C) store_row_f32(rs, (unsigned)((c * cstride + (size_t)n * 4) * sizeof(R)), y[c]);
+    } else {
+      R* p = base + (size_t)(v - a.T) * sstride;
+#pragma unroll
+      for (int c = 0; c < CM; ++c)
+        if (EXACT || c < C) st4(p + (size_t)c * cstride, y[c]);
+    }
     est[so * 64 + lane] = E;
     e0 = f0;
     e1 = f1;
