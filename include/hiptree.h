@@ -88,9 +88,9 @@ int hx_plan_info(hx_plan_t plan, int* post_levels, int* pre_levels, int* max_wid
 
 /* The four-state walk programs of a plan (no reference counterpart: accounting of what
  * the walks move): post-order stack entries, pre-order stack depth, cherries (internal
- * nodes whose children are both tips), and the cherries whose partial the post-order walk
- * does not store under register mode 0 and 1 (rebuilt by the pre-order walk). Any output
- * pointer may be NULL. */
+ * nodes whose children are both tips), and the cherries whose partial the FP32 post-order walk
+ * does not store (rebuilt by the pre-order walk; both outputs: the walk has one mode). Any
+ * output pointer may be NULL. */
 int hx_plan_walk_info(hx_plan_t plan, int* post_need, int* pre_depth, int* cherries,
                       int* dropped_mode0, int* dropped_mode1);
 

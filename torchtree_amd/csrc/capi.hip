@@ -96,9 +96,8 @@ int hx_plan_create(int taxa, const int32_t* postorder, int device, hx_plan_t* ou
     pre_lv[depth[v]].push_back(v);
   }
   std::vector<int32_t> walk, segtab;
-  std::vector<uint8_t> drop;
   int walk_need = 0;
-  if (!hx::build_walk(T, kids, postorder, walk, segtab, walk_need, &drop)) {
+  if (!hx::build_walk(T, kids, postorder, walk, segtab, walk_need)) {
     hx::set_error("walk program construction failed");
     return HX_ERR_BAD_TOPOLOGY;
   }
@@ -161,10 +160,7 @@ int hx_plan_create(int taxa, const int32_t* postorder, int device, hx_plan_t* ou
   plan->d_pre4 = plan->d_buf + pre4_off;
   plan->post4_slots = post4_slots;
   plan->ncher = (int)(cher.size() / 2);
-  for (uint8_t b : drop) {
-    plan->ndrop[0] += b & 1;
-    plan->ndrop[1] += (b >> 1) & 1;
-  }
+  plan->ndrop = (int)std::count(drop4.begin(), drop4.end(), 1);
   *out = plan;
   return HX_OK;
 }
@@ -182,8 +178,8 @@ int hx_plan_walk_info(hx_plan_t plan, int* post_need, int* pre_depth, int* cherr
   if (post_need) *post_need = plan->walk_need;
   if (pre_depth) *pre_depth = plan->prew_depth;
   if (cherries) *cherries = plan->ncher;
-  if (dropped_mode0) *dropped_mode0 = plan->ndrop[0];
-  if (dropped_mode1) *dropped_mode1 = plan->ndrop[1];
+  if (dropped_mode0) *dropped_mode0 = plan->ndrop;
+  if (dropped_mode1) *dropped_mode1 = plan->ndrop;
   return HX_OK;
 }
 

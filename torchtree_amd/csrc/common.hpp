@@ -62,7 +62,7 @@ struct hx_plan_s {
   const int32_t* d_post4 = nullptr;
   const int32_t* d_pre4 = nullptr;
   int post4_slots = 0;
-  // Cherries, and how many build_walk's drop bits name under register mode 0 and 1.
+  // Cherries, and how many of them the four-state FP32 walks leave out of memory (build_post4).
   int ncher = 0;
-  int ndrop[2] = {0, 0};
+  int ndrop = 0;
 };
