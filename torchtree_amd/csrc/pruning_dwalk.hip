@@ -372,7 +372,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 #pragma unroll
       for (int r = 0; r < 4; ++r) est[((cur.m >> 16) & 0xff) * kTile + 4 * g + r] = E[r];
     }
-    if (STORE || spill) d.store_acc(d.node(cur.v, true), y);
+    if ((STORE && i + 1 < nprog) || spill) d.store_acc(d.node(cur.v, true), y);
     cur = nxt;
   };
   for (int i = 0; i < nprog; ++i) {

@@ -280,7 +280,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const bool spill = (e.m >> 4) & 1;
     if (spill) est[((e.m >> 16) & 0xff) * 64 + lane] = E;
     if (STORE || spill) {
-      const bool empty = ((e.m >> 3) & 1) && a.drop;
+      const bool empty = (((e.m >> 3) & 1) && a.drop) || i + 1 == nprog;  // (the root's: never read)
       const auto r = node_buf(e.v, empty ? 0 : nbytes);
 #pragma unroll
       for (int c = 0; c < CM; ++c)
