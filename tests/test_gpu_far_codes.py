@@ -15,6 +15,7 @@ def test_codes_past_4_gib(gpu):
 
     T, n, times, S = 2100, 1024, 2002, 4
     assert T * n * times > 1 << 32
+    torch.cuda.empty_cache()
     if torch.cuda.mem_get_info(gpu)[0] < 130 << 30:
         pytest.skip("needs 130 GiB of device memory")
     g = torch.Generator(device=gpu).manual_seed(1)

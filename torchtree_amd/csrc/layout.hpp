@@ -164,9 +164,9 @@ inline bool use_nat_rows(int S, int C) {
 //          20 in 16-byte loads, the other sizes word by word, and rows of a multiple of 8 states
 //          (past 20; of 16 with several categories) fall on the same banks.
 //   levels (launch) x levels + I B C v.
-// Measured at 15 state counts of 2 to 32, 1 to 4 categories, 8 to 350 taxa (caterpillars to balanced
-// trees), 1 to 100000 patterns and 1 to 32 samples, 7092 calls: the faster one is chosen but for
-// 65 that lose 10 to 42 %; with the walk everywhere 350 taxa x 60 patterns, 27 states, 4 categories
+// Measured at 12 state counts of 2 to 32, 1 to 4 categories, 8 to 350 taxa (caterpillars to balanced
+// trees), 1 to 100000 patterns and 1 to 32 samples, 7870 calls: the slower one costs more than 10 % in
+// 59 of them (at most 42 %); with the walk everywhere 350 taxa x 60 patterns, 27 states, 4 categories
 // took 1068 us (levels 112), 128 x 400 at 20 states 163 (60).
 constexpr int kDwalkMaxS = 32;
 inline bool use_dwalk(int S, int C, int I, int levels, int ntiles, int K) {
@@ -177,8 +177,8 @@ inline bool use_dwalk(int S, int C, int I, int levels, int ntiles, int K) {
   else if (S < 20) a = 0.8 + 0.27 * C, b = 0.0009;
   else if (S == 20) a = 0.84 + 0.1 * C, b = 0.0006;
   else a = 0.95 + 0.47 * C, b = S % 8 == 0 ? 0.003 : 0.0019;
-  const double launch = S <= 16 ? 4.25 + 0.1 * C : 4.7 + 0.22 * C;
-  const double v = S <= 16 ? 0.00067 : (S <= 20 ? 0.00115 : 0.0016);
+  const double launch = S <= 16 ? 4.0 + 0.08 * C : (S <= 20 ? 3.95 + 0.37 * C : 4.7 + 0.22 * C);
+  const double v = S <= 16 ? 0.00065 : (S <= 20 ? (C < 4 ? 0.0014 : 0.00115) : 0.0016);
   return 8 + I * (a + b * C * past) <= levels * launch + I * blocks * C * v;
 }
 
