@@ -62,10 +62,10 @@ inline int wide_nt(int C, int S, int rb) {
 // S == 4 uses tiles of 64 patterns (a wave per category, a lane per pattern);
 // other S use tiles of wide_nt() patterns handled by (child, category, state)
 // lanes.
-// The chunking and the kernels depend on N, S, the precision and the tile shape only, never
-// on K: a sample's
+// The chunking depends on N, S, C, the precision and the tile shape only, never on K: a sample's
 // sums run in the same order whatever batch it is evaluated in, so its result is bitwise
-// identical alone and in a batch.
+// identical alone and in a batch. (K enters post_level_tiles and use_dwalk, which no result
+// depends on.)
 constexpr int kTargetChunks = 128;
 
 // The four-state FP32 passes with at most kPreWalkMaxC categories are walks

@@ -1,5 +1,6 @@
 // Dense-state FP32 post-order (S != 4, at most 32 states and 4 categories) as one walk: a launch for
-// the whole tree.
+// the whole tree, for the calls that use_dwalk (layout.hpp) gives it: with few patterns on a large
+// tree the level kernels are ahead. The partials and root sums are theirs to the bit.
 //
 // Reference: calculate_treelikelihood_discrete* (torchtree/evolution/tree_likelihood.py:40-278)
 // at S != 4.
@@ -19,8 +20,7 @@
 // child back from memory and leaves the chip nearly empty at the narrow levels (about 30 us each).
 // Measured against it, 20 states, 4 categories, FP32: 256 taxa x 20000 patterns 1815 -> 1005 us,
 // 173 taxa x 3203 patterns at 8 samples 1495 -> 900 us; with split-BF16 products at the first size
-// 1747 -> 1000 us (each operand is split when it is used; their products are those of the level
-// kernels, to the bit). Past 32 states the operands of two children's matrices no longer fit a
+// 1747 -> 1000 us (each operand is split when it is used). Past 32 states the operands of two children's matrices no longer fit a
 // wave's registers (61 states: 64 x 2, fetched a node ahead).
 #include "pruning.hpp"
 #include "split.hpp"

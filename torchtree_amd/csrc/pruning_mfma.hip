@@ -339,8 +339,8 @@ struct FwdP {
 }  // namespace
 
 // ---------------------------------------------------------------- post-order
-// Launched for the root (ROOT = true: the per-chunk root sums of loglik, d/dfreqs
-// and d/dprops); the levels below use k_post_mfma_r.
+// Launched for the root (ROOT = true: the root sums of loglik, d/dfreqs and d/dprops, of each of
+// its parts); the levels below use k_post_mfma_r.
 template <typename R, int MT, int KV, int TIPS, bool ROOT, bool SPLIT = false>
 __global__ __launch_bounds__(512) void k_post_mfma(PassArgs<R> a,
                                                    const int32_t* __restrict__ nodes, int S) {
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
   R* Yx = reinterpret_cast<R*>(smem_raw);              // [C][16][LS] child-1 products
   R* mx = Yx + C * kTile * LS;                         // [16][4] per-row category maxima
   int* Et = reinterpret_cast<int*>(mx + 4 * kTile);    // [2 parity][2 children][16]
-  // FP32: the wave's tile of child rows (its product tile, for h = 1: see the barriers)
+  // NAT: the wave's tile of child rows (its product tile, for h = 1: see the barriers)
   constexpr bool kNat = NAT;
   R* Lt = reinterpret_cast<R*>(Et + 4 * kTile);        // [C][16][LS]
 
@@ -556,7 +556,7 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
   const float qmask = chq >= a.T ? 1.f : 0.f;
   lds_barrier();
 
-  // FP64: a tile's child rows as operands (rows clamped to N - 1, states past S read the row's
+  // not NAT: a tile's child rows as operands (rows clamped to N - 1, states past S read the row's
   // last state; both are zeroed with a select when the tile starts)
   auto post_rows = [&](int tl, int code, R (&row)[KV]) {
     const int ncl = min(tl * kTile + nn, a.N - 1);
@@ -586,7 +586,7 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
 #pragma unroll
     for (int q = 0; q < KV; ++q) row[q] = bp[min(base + q, last)];
   };
-  // a tip's codes are on their way for the time of a tile, and so are FP32's rows
+  // a tip's codes are on their way for the time of a tile, and so are NAT's rows
   const bool coded = TIPS == HX_TIPS_CODES && !internal;
   const uint8_t* tcodes = coded ? a.codes + (size_t)chh * a.N : nullptr;
   auto code_of = [&](int tl) -> int { return coded ? tcodes[min(tl * kTile + nn, a.N - 1)] : 0; };
@@ -1469,8 +1469,7 @@ template <typename R>
 static size_t mfma_lds(int C, int S, bool pre) {
   const int MT = S <= 16 ? 1 : (S <= 32 ? 2 : 4);
   const size_t SP = 16 * MT, rb = sizeof(R);
-  // k_pre_mfma_r (MT <= 2) pads the per-row category entries to 4 and stages
-  // two children's codes for the chunk
+  // k_pre_mfma_r pads the per-row category entries to 4
   if (pre && (MT <= 2 || rb == 4)) {
     const int KV = MT == 2 && S <= 20 ? 5 : 4 * MT;
     const size_t pt = MT <= 2 ? 2 * (size_t)C * 4 * KV * (SP + 1) : 0;  // transpose P tiles
@@ -1489,8 +1488,8 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   const int threads = 2 * a.C * 64;
   const size_t lds = mfma_lds<R>(a.C, S, !post);
   const bool nat = sizeof(R) == 4 && use_nat_rows(S, a.C);
-  // LDS holds no codes of a chunk any more, and its rows are padded at 64 states; a chunk too large
-  // for the codes stays refused
+  // the kernels stage no codes; a chunk whose codes would not fit beside unpadded tiles is refused as
+  // it was when they did
   const size_t codes = 2 * (size_t)a.tiles_per_chunk * kTile;
   const size_t tilef = (size_t)a.C * kTile * (16 * MT + 4);
   const size_t pads = (sizeof(R) == 4 ? tilef * sizeof(R) : 0) +

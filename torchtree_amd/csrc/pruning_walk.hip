@@ -19,14 +19,14 @@
 // samples) the stores of the post-order and the LDS and issue slots of the pre-order. P used to
 // sit in scalar registers, whose loads return out of order, so that each category of each node
 // waited for a scalar-cache miss (about 0.5 us); as vector loads, counted in order, they run
-// ahead. Measured against that, the whole call: 60 taxa x 431 patterns, 8 samples, d/dtau: 337 -> 158
-// us; 413 x 9,871, 8 samples, d/dtau: 2.70 -> 1.40 ms; 512 x 20,011, 4 samples, log-likelihood alone:
-// 1.14 -> 0.33 ms; 512 x 100,000, 32 samples, d/dP: 56.4 -> 48.2 ms (post-order 20.2 -> 15.3 ms,
-// pre-order 33.9 -> 31.5 ms).
+// ahead. Measured against that, the whole call: 60 taxa x 431 patterns, 8 samples, d/dtau: 337 -> 187
+// us; 413 x 9,871, 8 samples, d/dtau: 2.72 -> 1.55 ms; 512 x 20,011, 4 samples, log-likelihood alone:
+// 1.13 -> 0.33 ms; 512 x 100,000, 32 samples, d/dP: 55.9 -> 47.4 ms (post-order 20.2 -> 14.8 ms,
+// pre-order 33.9 -> 31.7 ms).
 //
 // Tried here and slower: categories across lanes instead of registers (16 to 64 patterns per wave,
-// the statistic's transposes as products with the identity): 413 x 9,871 1.65-2.1 ms against 1.41,
-// 512 x 100,000 58-77 ms against 48.6; a load around which the program branches (the register
+// the statistic's transposes as products with the identity; d/dtau then in FP32 per pattern on both
+// sides): 413 x 9,871 1.65-2.1 ms against 1.41, 512 x 100,000 58-77 ms against 48.6; a load around which the program branches (the register
 // copies that join the two paths wait for it at once): the pre-order walks +8 %.
 #include "pruning.hpp"
 #include "walk.hpp"
@@ -148,8 +148,8 @@ __device__ __forceinline__ unsigned p_offset(int lane, int C, bool trans) {
 // so the waits count loads exactly and never a recent store. The program itself comes in blocks of
 // 16 entries, one word per lane, read by v_readlane: no scalar load is outstanding when the
 // tip table is read from LDS (the two share a counter, and scalar loads return out of order).
-// STORE: a gradient may follow, so every internal partial but the dropped cherries' is stored;
-// otherwise (the workspace has no room for one) only spilled results are.
+// STORE: a gradient may follow, so every internal partial but the dropped cherries' and the root's
+// is stored; otherwise (hx_loglik_value) only spilled results are.
 // grid = (ntiles, ceil(K / W)), block = 64 W.
 constexpr int kAhead = 3;
 

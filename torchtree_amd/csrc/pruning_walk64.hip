@@ -341,8 +341,8 @@ k_post_walk64(PassArgs<double> a, const int* __restrict__ prog, int nprog, int s
 // waves per SIMD; the matrix cores are busy 11 % of it at 100,000 patterns. Kernel and sum, against a
 // launch per level (k_pre) that read and wrote every adjoint: 64 taxa x 100000 patterns, 4
 // categories 858 -> 503 us; 100 x 3000 at 8 samples, d/dtau 552 -> 218; 64 x 997, one category 70 ->
-// 51; 211 x 5003 270 and 15 launches'
-// gaps -> 292 (by level: runs_pre_walk64, pruning.hip).
+// 51; 211 x 5003 270 and 15 launches' gaps -> 292 (a tree of fewer levels goes by level:
+// runs_pre_walk64, pruning.hip).
 // Slower: partials and matrices in strided loads (820, 366 and 460 us of the three with 4
 // categories), tips looked up an entry ahead without branches (+3 %); the same: one buffer for a
 // node's categories.

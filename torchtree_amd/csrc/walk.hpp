@@ -28,7 +28,9 @@
 // Tips are consumed in walk order; consecutive entries are grouped into
 // segments of at most kWalkSegTips tips so a kernel can stage the codes of
 // one segment while it works through the previous one. segtab holds
-// kWalkSegTips tip ids per segment (-1 padding).
+// kWalkSegTips tip ids per segment (-1 padding). The kernels read [0]..[3] and
+// [6] only: they load codes entries ahead instead of staging them, and take
+// which cherries stay out of memory from build_post4.
 #pragma once
 
 #include <algorithm>
