@@ -360,17 +360,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // All of an entry's loads are issued in the entry before it, ahead of that entry's store (the
 // adjoint it pushes, which the next entry never pops); an empty range reads nothing.
 //
-// G: each wave writes Ut (rows 4c + i) and (w / lik) L (rows 4c + j) to LDS, pattern minor, and
-// reads them back as the operands of 16 v_mfma_f32_4x4x1_16b_f32, whose block 4c + q sums
-// category c's 4 x 4 outer products over patterns 16q .. 16q + 15; row rotations add the four
-// blocks q. The W waves' G meet in LDS one entry later (one barrier per entry, two buffers).
+// G: each wave writes (w / lik) Ut (rows 4c + i) and L (rows 4c + j) to LDS, pattern minor, and
+// reads them back as the operands of 4 CM v_mfma_f32_4x4x1_16b_f32, whose blocks share the patterns
+// of a category out: block (16 / CM) c + q sums its 4 x 4 outer products over 4 CM of them. Row
+// rotations add four blocks; what is left of a category (4 / CM rows of 16 lanes) and the W waves'
+// G meet in LDS one entry later (one barrier per entry, two buffers). With rows and products for
+// four categories whatever their number (56 KB of LDS: 2 waves per SIMD) the calls of one category
+// were behind a walk on the vector units, 64 taxa x 400,000 patterns, 4 samples, a caterpillar, d/dP:
+// 1294 us against 1651 (1166 now); 256 x 100,000, 2 samples, 2 categories, d/dP: 1315 -> 1061.
 //
 // dtau: the 16 sums of a (child, category) meet dP/dtau in FP64 on their way out. Rows of dP/dtau sum
 // to zero, so this contraction cancels. Done in FP32, per pattern and ahead of the sums, it needs no
 // transposes, but its error against 64 bits was 1.04 to 1.1 times as large (the calls 60 taxa x 431
 // patterns and 413 x 9871 at 8 samples took 135 and 1380 us so, 164 and 1504 as here); in FP64 per
 // pattern they took 177 and 1854.
-constexpr int kXS = 68;  // row stride (floats) of the LDS pattern transposes
+//
+// Row stride (floats) of the LDS pattern transposes, and where a block's patterns lie: with four
+// categories 16 running ones, with fewer fours 64 / CM apart. Either way the 16-byte reads of 16
+// lanes (4 rows, 4 blocks) fall on different banks.
+constexpr int xs_stride(int CM) { return CM == 4 ? 68 : 80; }
 
 // v + (v from the lane `ROT` below in the same row of 16 lanes, cyclically): DPP row_ror
 template <int ROT>
@@ -379,13 +387,18 @@ __device__ __forceinline__ float add_row_ror(float v) {
   return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v),
                                                                  0x120 + ROT, 0xF, 0xF, true));
 }
-constexpr size_t kPre4LdsFloats = (size_t)kPreWalkW * 3 * 16 * kXS + 4 * kPreWalkW * 64;
+constexpr size_t pre4_lds_floats(int CM) {
+  return (size_t)kPreWalkW * 3 * 4 * CM * xs_stride(CM) + 4 * kPreWalkW * 64;
+}
 
 template <int TIPS, int CM, bool EXACT, bool TAU>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CM == 4 ? 2 : 3))) void
 k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __restrict__ mats_dt,
             const int* __restrict__ prog, int nprog) {
   constexpr int W = kPreWalkW;  // waves (tiles) per workgroup
+  constexpr int RW = 4 * CM;    // rows of a transposed set
+  constexpr int RC = 4 / CM;    // rows of 16 lanes per category
+  constexpr int kXS = xs_stride(CM);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int C = EXACT ? CM : a.C;
   const int wave = uni(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -397,11 +410,11 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
   const int n = tl * 64 + lane;
   const bool val = tval && n < a.N;
   float* sm = reinterpret_cast<float*>(smem_raw);
-  float* xs = sm + (size_t)wave * 3 * 16 * kXS;  // rows 4c + i: (w / lik) Ut[c][i] of one child
-  float* ls = xs + 16 * kXS;                     // [2] rows 4c + j: L[c][j] (a tip: rows j)
-  float* red = sm + (size_t)W * 3 * 16 * kXS;    // [2][2][W][64]
-  f4* tbl = reinterpret_cast<f4*>(sm + kPre4LdsFloats);
-  for (int i = lane; i < 3 * 16 * kXS; i += 64) xs[i] = 0.f;  // rows of absent categories
+  float* xs = sm + (size_t)wave * 3 * RW * kXS;  // rows 4c + i: (w / lik) Ut[c][i] of one child
+  float* ls = xs + RW * kXS;                     // [2] rows 4c + j: L[c][j] (a tip: rows j)
+  float* red = sm + (size_t)W * 3 * RW * kXS;    // [2][2][W][64]
+  f4* tbl = reinterpret_cast<f4*>(sm + pre4_lds_floats(CM));
+  for (int i = lane; i < 3 * RW * kXS; i += 64) xs[i] = 0.f;  // rows of absent categories
   stage_table<TIPS>(a, tbl);
 
   const float w = val ? (float)a.weights[n] : 0.f;
@@ -506,7 +519,10 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
     if ((int)threadIdx.x < 2 * CS) {
       float s = 0.f;
 #pragma unroll
-      for (int q = 0; q < W; ++q) s += red[((par * 2 + sh) * W + q) * 64 + se];
+      for (int q = 0; q < W; ++q)
+#pragma unroll
+        for (int r = 0; r < RC; ++r)
+          s += red[((par * 2 + sh) * W + q) * 64 + (RC * (se >> 4) + r) * 16 + (se & 15)];
       const size_t at = ((size_t)(sh ? b2 : b1) * a.K + k) * a.nchunks + chunk;
       if constexpr (TAU) {
         double t = (double)(s * spc) * (double)dp;
@@ -558,7 +574,7 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
         else t = x.t[h];
         mv4<CM>(x.p[h], [&](auto) { return t; }, m[h]);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) ls[(16 * h + s) * kXS + lane] = t[s];
+        for (int s = 0; s < 4; ++s) ls[(RW * h + s) * kXS + lane] = t[s];
       } else {
         if constexpr (TIPS == HX_TIPS_CODES) {
           if (kd == 1) {
@@ -578,7 +594,7 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
         for (int c = 0; c < CM; ++c)
           if (EXACT || c < C)
 #pragma unroll
-            for (int s = 0; s < 4; ++s) ls[(16 * h + 4 * c + s) * kXS + lane] = L[c][s];
+            for (int s = 0; s < 4; ++s) ls[(RW * h + 4 * c + s) * kXS + lane] = L[c][s];
       }
       __builtin_amdgcn_sched_barrier(0);  // one child's registers at a time
     });
@@ -601,11 +617,12 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
     }
     auto Ut = [&](auto hc) -> f4(&)[CM] { return m[1 - decltype(hc)::value]; };
     const float coef = (val && lik > 0.f) ? w * __builtin_amdgcn_rcpf(lik) : 0.f;
-    // Block b = 4c + q of the 4x4x1 product: lane 4b + i gives A[b][i] = (w / lik) Ut[c][i] and
-    // lane 4b + j gives B[b][j] = L[c][j] of pattern 16q + m in product m; register i of lane
+    // Block b = (16 / CM) c + q of the 4x4x1 product: lane 4b + i gives A[b][i] = (w / lik) Ut[c][i]
+    // and lane 4b + j gives B[b][j] = L[c][j] of the block's pattern m in product m; register i of lane
     // 4b + j accumulates G[c][i][j] over those patterns. Child 2's Ut rows overwrite child 1's
     // after child 1's operand reads (LDS operations of a wave stay in order).
-    const int g4 = lane >> 4, srow = 4 * g4 + (lane & 3), scol = 16 * ((lane >> 2) & 3);
+    const int g4 = lane >> 4, srow = 4 * (g4 / RC) + (lane & 3);
+    const int scol = (CM == 4 ? 16 : 4) * ((lane >> 2) % (16 / CM));
     auto stat_rows = [&](auto hc) {
 #pragma unroll
       for (int c = 0; c < CM; ++c)
@@ -615,12 +632,13 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
     };
     auto stat_mfma = [&](int h) {
       __builtin_amdgcn_wave_barrier();
-      const int rl = 16 * h + (kind(m_, h) == 0 ? (lane & 3) : srow);
+      const int rl = RW * h + (kind(m_, h) == 0 ? (lane & 3) : srow);
       f4 g[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const f4 A = *reinterpret_cast<const f4*>(xs + srow * kXS + scol + 4 * u);
-        const f4 Bv = *reinterpret_cast<const f4*>(ls + rl * kXS + scol + 4 * u);
+      for (int u = 0; u < CM; ++u) {
+        constexpr int US = CM == 4 ? 4 : 64 / CM;
+        const f4 A = *reinterpret_cast<const f4*>(xs + srow * kXS + scol + US * u);
+        const f4 Bv = *reinterpret_cast<const f4*>(ls + rl * kXS + scol + US * u);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           g[e & 1] = __builtin_amdgcn_mfma_f32_4x4x1f32(A[e], Bv[e], g[e & 1], 0, 0, 0);
@@ -628,12 +646,12 @@ k_pre_walk4(PassArgs<float> a, const float* __restrict__ mats, const float* __re
       __builtin_amdgcn_wave_barrier();
       return g[0] + g[1];
     };
-    // The four pattern groups of each category (lanes 16c + 4q + j) are added by row rotations;
-    // lane 16c + j then holds G_h[c][i][j] in register i and writes it to the wave's slot.
+    // The four blocks of a row of 16 lanes are added by row rotations; lane 16 r + j then holds row
+    // r's share of G_h[r / RC][i][j] in register i and writes it to the wave's slot.
     auto stat_put = [&](int h, f4 g) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) g[r] = add_row_ror<8>(add_row_ror<4>(g[r]));
-      if (((lane >> 2) & 3) == 0 && g4 < C) {
+      if (((lane >> 2) & 3) == 0 && g4 < C * RC) {
         float* dst = red + (((i & 1) * 2 + h) * W + wave) * 64 + g4 * 16 + (lane & 3);
 #pragma unroll
         for (int r = 0; r < 4; ++r) dst[4 * r] = g[r];
@@ -725,7 +743,7 @@ int launch_pre_walk4(const PassArgs<float>& a, const int32_t* prog, int nprog, i
   HX_REQUIRE(a.C >= 1 && a.C <= kPreWalkMaxC && a.nchunks == (a.ntiles + kPreWalkW - 1) / kPreWalkW,
              HX_ERR_UNSUPPORTED, "pre-order walk: chunking does not match the workgroup's tiles");
   const bool tau = a.mats_dt != nullptr;
-  const size_t lds = kPre4LdsFloats * 4 + table_bytes(tips, a.ncodes);
+  const size_t lds = pre4_lds_floats(a.C <= 2 ? a.C : 4) * 4 + table_bytes(tips, a.ncodes);
   HX_REQUIRE(lds <= 64 * 1024, HX_ERR_UNSUPPORTED, "pre-order walk: LDS");
   const auto kern = a.C == 1   ? pre_kernel<1, true>(tips, tau)
                     : a.C == 2 ? pre_kernel<2, true>(tips, tau)
