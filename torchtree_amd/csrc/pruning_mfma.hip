@@ -994,7 +994,8 @@ constexpr int kPD = 4;
 // Same products and barriers as k_pre_mfma.
 template <typename R, int MT, int KV, int TIPS, bool ROOT, bool SPLIT, bool NAT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
-    sizeof(R) == 4 && MT <= 2 ? (SPLIT && KV == 8 ? 3 : 4) : 1))) void k_pre_mfma_r(
+    sizeof(R) == 4 && MT <= 2 ? (SPLIT && KV == 8 ? 3 : 4)
+                              : (sizeof(R) == 8 && MT == 1 ? 5 : 1)))) void k_pre_mfma_r(
     PassArgs<R> a, const int32_t* __restrict__ nodes, int S) {
   static_assert(MT <= 2 || (sizeof(R) == 4 && KV == 16), "64 padded states: FP32, 16 steps");
   // split products: the statistic's L tile, the transpose's P tile and the padded P copies
@@ -1002,6 +1003,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   using SSh = SplitShape<KV>;
   constexpr int KB = SSh::KB, NB = SSh::NB;
   constexpr bool kPReg = MT <= 2;
+  // FP64 up to 16 states runs at 5 waves per SIMD, which needs a tip's code loaded ahead of its rows,
+  // the rows masked before the adjoint's loads and the weights' loads last (8 states, 2 categories, 50
+  // taxa x 20000 patterns at 8 samples: 100 registers and 2352 us otherwise)
+  constexpr bool kTight = sizeof(R) == 8 && MT == 1;
   constexpr int SP = 16 * MT;
   // LDS row stride of the [16][SP] tiles: SP + 4 starts rows 4g + r of the accumulator layout 16g
   // banks apart (SP puts the four lane groups g, and an operand's 16 rows, on the same banks)
@@ -1157,9 +1162,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
       if constexpr (!ROOT && kNatU && !kPReg) urows.load(tl, h * NU, 0, un);
       if constexpr (!kPReg) load_wt(tl, wtn);
     } else {
-      pre_rows<R, KV, TIPS>(a, internal, cslab, chh, code, tl, nn, g, S, CS, cb, arow);
+      const int now = code;
+      if constexpr (kTight) code = code_of(min(tl + 1, t1 - 1));
+      pre_rows<R, KV, TIPS>(a, internal, cslab, chh, now, tl, nn, g, S, CS, cb, arow);
     }
-    code = code_of(min(tl + 1, t1 - 1));
+    if constexpr (!kTight) code = code_of(min(tl + 1, t1 - 1));
   };
   next_rows(t0);
   // the parent's adjoint (zero past N and S) of a tile in the accumulator layout
@@ -1187,6 +1194,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   for (int tile = t0; tile < t1; ++tile) {
     const int nbase = tile * kTile;
     const uint32_t tb = (uint32_t)nbase * (uint32_t)CS;
+    if constexpr (kTight) pre_rows_mask<R, KV>(a.N, tile, nn, g, S, arow);
     bool rok[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) rok[r] = nbase + acc_row<R>(g, r) < a.N;
@@ -1195,7 +1203,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     if constexpr (kNat && !kPReg) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) wt[r] = wtn[r];
-    } else {
+    } else if constexpr (!kTight) {
       load_wt(tile, wt);
     }
     if constexpr (kNatU && !ROOT) {
@@ -1203,6 +1211,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     } else {
       load_up(tile, up);
     }
+    if constexpr (kTight) load_wt(tile, wt);
 
     // forward P_h L_h; the tile of L is kept as the statistic's B operand
     vec4_t<R> acc[MT];
@@ -1219,7 +1228,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
       }
       lds_run<KV>(lt + nn * LS + g * KV, ow);
     } else {
-      pre_rows_mask<R, KV>(a.N, tile, nn, g, S, arow);
+      if constexpr (!kTight) pre_rows_mask<R, KV>(a.N, tile, nn, g, S, arow);
 #pragma unroll
       for (int q = 0; q < KV; ++q) {
         if constexpr (SPLIT) ow[q] = __builtin_bit_cast(float, bf_pair(arow[q]));
