@@ -61,3 +61,12 @@ def test_tau_chunks_grow_with_the_patterns(ask):
     assert ask([("tau", 77, 4, 9), ("tau", 188, 4, 9), ("tau", 500, 4, 9), ("tau", 1000, 4, 8),
                 ("tau", 5000, 1, 40), ("tau", 188, 1, 9), ("tau", 500, 1, 9), ("tau", 7, 4, 7),
                 ("tau", 1, 1, 1)]) == [5, 6, 8, 8, 40, 5, 6, 5, 1]
+
+
+@pytest.mark.parametrize("S", [33, 61, 64])
+def test_post_level_tiles_of_one_category_stay_short(ask, S):
+    """One category at 33 states and more: at most 10 tiles a block, whatever the launch holds."""
+    grid = [("tiles", S, nt, 1, K, w, f) for nt in (1, 7, 100, 1250, 6250, 65536) for K in (1, 8, 32)
+            for w in (1, 9, 64) for f in (0, 1)]
+    for q, t in zip(grid, ask(grid)):
+        assert 1 <= t <= min(q[2], 10), q

@@ -117,7 +117,13 @@ inline Tiling make_tiling(int N, int C, int K, int S, int rb) {
 // loads in the lane order of its operand), and blocks beyond a round of the chip wait for the next:
 // in the chunks of the gradient (8 tiles and more) the narrow levels near the root had 9 to 70 blocks
 // a sample, and others a nearly empty last round (61 states, 128 taxa x 10000 patterns, split
-// products: 1104 -> 968 us; FP32, 97 x 1217 at 8 samples: 1201 -> 984).
+// products: 1104 -> 968 us; FP32, 97 x 1217 at 8 samples: 1201 -> 984). `waves` is how many of the
+// kernel a SIMD holds: 2, or 3 with FP32 products and coded tips, and with 1 or 2 categories more
+// blocks of 2 C waves share a CU. (With 3 categories a third per SIMD gained nothing: blocks of 6
+// waves.) At one category rounds are long and blocks leave them one by one, and past 10 tiles a longer
+// chunk only coarsens the end: 33 to 61 states, 50 taxa x 20000 patterns at 8 samples, in percent
+// behind the best of 2 to 48 tiles: FP32 9 to 11 (2 categories 6 to 11), FP64 6 to 7, split 5, with
+// rounds of 1024 blocks and up to 64 tiles; 0 to 2 now.
 //
 // Below, blocks share a CU and hide each other's latency, and rounds of one block per CU leave it
 // idle. There a level takes about (blocks / 256 + tail) (t + set-up), least at t ~ sqrt(tiles C) with
@@ -126,17 +132,17 @@ inline Tiling make_tiling(int N, int C, int K, int S, int rb) {
 // them at most and mostly ahead; rounds of one block per CU were 0 to 73 % behind. FP64, 2 states, 4
 // categories, 50 taxa x 3000 patterns at 8 samples: 570 us in such rounds, 348 in the gradient's
 // chunks, 333 now; 20 states, 128 x 20000: 1773 in such rounds, 1556 now.
-inline int post_level_tiles(int ntiles, int S, int C, int K, int width, bool f64) {
+inline int post_level_tiles(int ntiles, int S, int C, int K, int width, bool f64, int waves = 2) {
   if (S <= 32) {
     const double q = S <= 16 ? 4096.0 : (S <= 20 && C <= 2 ? 2048.0 : 1024.0);
     const double t = sqrt((double)ntiles * K * width * C / q);
     const int nch = (int)(ntiles / (t < 1.0 ? 1.0 : t) + 0.5), least = (ntiles + 63) / 64;
     return (ntiles + (nch > least ? nch : least) - 1) / (nch > least ? nch : least);  // even chunks
   }
-  const double setup = f64 ? 4.0 : 1.0, slots = 256.0 * (C >= 4 ? 1 : 4 / C);
+  const double setup = f64 ? 4.0 : 1.0, slots = 256.0 * (C <= 2 ? 2 * waves / C : 1);
   int best = 1;
   double cost = 0.0;
-  for (int t = 1; t <= ntiles && t <= 64; ++t) {
+  for (int t = 1; t <= ntiles && t <= (C == 1 ? 10 : 64); ++t) {
     const double blocks = (double)((ntiles + t - 1) / t) * K * width;
     const double c = ceil(blocks / slots) * (t + setup);
     if (t == 1 || c <= cost) best = t, cost = c;

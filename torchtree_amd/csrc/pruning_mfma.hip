@@ -1547,7 +1547,8 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
     // (at most 36 KiB)
     const size_t lds_r = lds_b + (sizeof(R) == 4 ? (size_t)a.C * kTile * (16 * MT + 4) * 4 : 0);
     PassArgs<R> b = a;
-    b.tiles_per_chunk = post_level_tiles(a.ntiles, S, a.C, a.K, width, sizeof(R) == 8);
+    b.tiles_per_chunk = post_level_tiles(a.ntiles, S, a.C, a.K, width, sizeof(R) == 8,
+                                         sizeof(R) == 4 && !SPLIT && tips == HX_TIPS_CODES ? 3 : 2);
     grid.x = (a.ntiles + b.tiles_per_chunk - 1) / b.tiles_per_chunk;
 #define HX_MFR(MTV, KVV, NATV)                                                               \
   if (tips == HX_TIPS_CODES)                                                                 \
