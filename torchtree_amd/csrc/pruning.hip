@@ -285,6 +285,7 @@ static PassArgs<R> make_args(const CallArgs& c) {
   a.ppad = use_ppad(c.S, c.dtype, c.grad_mode) ? reinterpret_cast<R*>(base + w.ppad) : nullptr;
   a.split = c.dtype == HX_F32_BF16X3;
   a.lanes = runs_pre_walk64(c);
+  a.root_parts = 1;
   a.drop = runs_walk4(c) && walk_drop_mode(c.S, c.C, c.N, c.K, c.dtype, c.tip_kind) >= 0;
   return a;
 }

@@ -36,6 +36,7 @@ struct PassArgs {
   // pre-order rebuilds it from the two tips' codes.
   int drop;
   int lanes;  // four-state FP64: partials in the lane order of the pre-order walk, which follows
+  int root_parts;  // dense states: parts of the root's sums that a block takes (k_post_mfma)
 };
 
 constexpr double kLn2 = 0.69314718055994530942;

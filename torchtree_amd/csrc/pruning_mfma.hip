@@ -340,7 +340,11 @@ struct FwdP {
 
 // ---------------------------------------------------------------- post-order
 // Launched for the root (ROOT = true: the root sums of loglik, d/dfreqs and d/dprops, of each of
-// its parts); the levels below use k_post_mfma_r.
+// its parts); the levels below use k_post_mfma_r. A part is a.tiles_per_chunk tiles; a block takes
+// a.root_parts of them in turn, so that P is set up once for the tiles that post_level_tiles gives a
+// block, and the sums stay the parts' (a block a part, 4 taxa x 50000 patterns at 8 samples, split
+// products: 24 states, 4 categories 1.20 of what chunks of 25 tiles with a sum each took, 0.97 so; 32
+// states, 2 categories 1.19 and 0.90).
 template <typename R, int MT, int KV, int TIPS, bool ROOT, bool SPLIT = false>
 __global__ __launch_bounds__(512) void k_post_mfma(PassArgs<R> a,
                                                    const int32_t* __restrict__ nodes, int S) {
@@ -376,122 +380,127 @@ __global__ __launch_bounds__(512) void k_post_mfma(PassArgs<R> a,
     pc = a.props[(size_t)k * a.props_ks + c];
   }
 
-  const int t0 = chunk * a.tiles_per_chunk;
-  const int t1 = min(t0 + a.tiles_per_chunk, a.ntiles);
-  for (int tile = t0; tile < t1; ++tile) {
-    const int nbase = tile * kTile;
-    if (threadIdx.x < 2 * kTile) {
-      const int hh = threadIdx.x / kTile, m = threadIdx.x - hh * kTile, n = nbase + m;
-      const int chq = hh ? ch1 : ch0;
-      Et[threadIdx.x] =
-          (n < a.N && chq >= a.T) ? a.scales[((size_t)(chq - a.T) * a.K + k) * a.N + n] : 0;
-    }
-    vec4_t<R> acc[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) acc[t] = vec4_t<R>{R(0), R(0), R(0), R(0)};
-    R arow[KV];
-    child_row<R, TIPS, KV>(a, chh, k, nbase + nn, c, g * KV, S, arow);
-    fp.product(arow, acc);
-    // lane (nn, g): acc[t][r] = Y[m = 4 g + r][i = 16 t + nn]
-    if (h == 1) {
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) Yx[(c * kTile + acc_row<R>(g, r)) * SP + 16 * t + nn] = acc[t][r];
-    }
-    lds_barrier();
-    R x[MT][4];
-    if (h == 0) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        R m_ = R(0);
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          x[t][r] = acc[t][r] * Yx[(c * kTile + acc_row<R>(g, r)) * SP + 16 * t + nn];
-          m_ = fmax_(m_, x[t][r]);
-        }
-        m_ = row_max16(m_);
-        if (nn == 0) mx[c * kTile + acc_row<R>(g, r)] = m_;
+  const int p1 = min((chunk + 1) * a.root_parts, a.nchunks);
+  for (int part = chunk * a.root_parts; part < p1; ++part) {
+    const int t0 = part * a.tiles_per_chunk, t1 = min(t0 + a.tiles_per_chunk, a.ntiles);
+    for (int tile = t0; tile < t1; ++tile) {
+      const int nbase = tile * kTile;
+      if (threadIdx.x < 2 * kTile) {
+        const int hh = threadIdx.x / kTile, m = threadIdx.x - hh * kTile, n = nbase + m;
+        const int chq = hh ? ch1 : ch0;
+        Et[threadIdx.x] =
+            (n < a.N && chq >= a.T) ? a.scales[((size_t)(chq - a.T) * a.K + k) * a.N + n] : 0;
       }
-    }
-    lds_barrier();
-    if (h == 0) {
+      vec4_t<R> acc[MT];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = acc_row<R>(g, r), n = nbase + m;
-        R M = R(0);
-        for (int cc = 0; cc < C; ++cc) M = fmax_(M, mx[cc * kTile + m]);
-        int e = 0;
-        if (M > R(0) && isfinite(M)) {
-          frexp_(M, &e);
+      for (int t = 0; t < MT; ++t) acc[t] = vec4_t<R>{R(0), R(0), R(0), R(0)};
+      R arow[KV];
+      child_row<R, TIPS, KV>(a, chh, k, nbase + nn, c, g * KV, S, arow);
+      fp.product(arow, acc);
+      // lane (nn, g): acc[t][r] = Y[m = 4 g + r][i = 16 t + nn]
+      if (h == 1) {
 #pragma unroll
-          for (int t = 0; t < MT; ++t) x[t][r] = ldexp_(x[t][r], -e);
-        }
-        const int E = Et[m] + Et[kTile + m] + e;
-        if constexpr (!ROOT) {
-          if (n < a.N) {
-            const size_t row = ((size_t)(v - a.T) * a.K + k) * a.N + n;
+        for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int t = 0; t < MT; ++t)
-              if (16 * t + nn < S) a.partials[(row * C + c) * S + 16 * t + nn] = x[t][r];
-            if (c == 0 && nn == 0) a.scales[row] = E;
+          for (int r = 0; r < 4; ++r) Yx[(c * kTile + acc_row<R>(g, r)) * SP + 16 * t + nn] = acc[t][r];
+      }
+      lds_barrier();
+      R x[MT][4];
+      if (h == 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          R m_ = R(0);
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            x[t][r] = acc[t][r] * Yx[(c * kTile + acc_row<R>(g, r)) * SP + 16 * t + nn];
+            m_ = fmax_(m_, x[t][r]);
           }
-        } else {
-          R p_ = R(0);
-#pragma unroll
-          for (int t = 0; t < MT; ++t) p_ = fma(pi_t[t], x[t][r], p_);
-          p_ = row_sum16(p_);
-          if (nn == 0) pxs[c * kTile + m] = (double)p_;
-          if (c == 0 && nn == 0) Er[m] = E;
+          m_ = row_max16(m_);
+          if (nn == 0) mx[c * kTile + acc_row<R>(g, r)] = m_;
         }
       }
-    }
-    if constexpr (ROOT) {
       lds_barrier();
       if (h == 0) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int m = acc_row<R>(g, r), n = nbase + m;
-          if (n >= a.N) continue;
-          double lik = 0.0;
-          for (int cc = 0; cc < C; ++cc)
-            lik += (double)(a.props[(size_t)k * a.props_ks + cc] * (R)pxs[cc * kTile + m]);
-          const double w = a.weights[n];
-          const double wi = w / lik;
-          if (c == 0 && nn == 0) acc_l += w * (log(lik) + (double)Er[m] * kLn2);
+          R M = R(0);
+          for (int cc = 0; cc < C; ++cc) M = fmax_(M, mx[cc * kTile + m]);
+          int e = 0;
+          if (M > R(0) && isfinite(M)) {
+            frexp_(M, &e);
 #pragma unroll
-          for (int t = 0; t < MT; ++t) acc_f[t] += wi * (double)(pc * x[t][r]);
-          if (nn == 0) acc_p += wi * pxs[c * kTile + m];
+            for (int t = 0; t < MT; ++t) x[t][r] = ldexp_(x[t][r], -e);
+          }
+          const int E = Et[m] + Et[kTile + m] + e;
+          if constexpr (!ROOT) {
+            if (n < a.N) {
+              const size_t row = ((size_t)(v - a.T) * a.K + k) * a.N + n;
+#pragma unroll
+              for (int t = 0; t < MT; ++t)
+                if (16 * t + nn < S) a.partials[(row * C + c) * S + 16 * t + nn] = x[t][r];
+              if (c == 0 && nn == 0) a.scales[row] = E;
+            }
+          } else {
+            R p_ = R(0);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) p_ = fma(pi_t[t], x[t][r], p_);
+            p_ = row_sum16(p_);
+            if (nn == 0) pxs[c * kTile + m] = (double)p_;
+            if (c == 0 && nn == 0) Er[m] = E;
+          }
         }
       }
-    }
-    lds_barrier();
-  }
-  if constexpr (ROOT) {
-    if (h == 0) {
+      if constexpr (ROOT) {
+        lds_barrier();
+        if (h == 0) {
 #pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        double f = acc_f[t];
-        f += __shfl_xor(f, 16);
-        f += __shfl_xor(f, 32);
-        if (g == 0) red[c * SP + 16 * t + nn] = f;
+          for (int r = 0; r < 4; ++r) {
+            const int m = acc_row<R>(g, r), n = nbase + m;
+            if (n >= a.N) continue;
+            double lik = 0.0;
+            for (int cc = 0; cc < C; ++cc)
+              lik += (double)(a.props[(size_t)k * a.props_ks + cc] * (R)pxs[cc * kTile + m]);
+            const double w = a.weights[n];
+            const double wi = w / lik;
+            if (c == 0 && nn == 0) acc_l += w * (log(lik) + (double)Er[m] * kLn2);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc_f[t] += wi * (double)(pc * x[t][r]);
+            if (nn == 0) acc_p += wi * pxs[c * kTile + m];
+          }
+        }
       }
-      acc_p += __shfl_xor(acc_p, 16);
-      acc_p += __shfl_xor(acc_p, 32);
-      acc_l += __shfl_xor(acc_l, 16);
-      acc_l += __shfl_xor(acc_l, 32);
+      lds_barrier();
     }
-    lds_barrier();
-    double* out = a.rootsums + ((size_t)k * a.nchunks + chunk) * (1 + S + C);
-    if (h == 0 && c == 0) {
-      for (int s = lane; s < S; s += 64) {
-        double tsum = 0.0;
-        for (int cc = 0; cc < C; ++cc) tsum += red[cc * SP + s];
-        out[1 + s] = tsum;
+    if constexpr (ROOT) {
+      // the part's sums (its readers of red are past it at the next tile's first barrier)
+      if (h == 0) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          double f = acc_f[t];
+          f += __shfl_xor(f, 16);
+          f += __shfl_xor(f, 32);
+          if (g == 0) red[c * SP + 16 * t + nn] = f;
+          acc_f[t] = 0.0;
+        }
+        acc_p += __shfl_xor(acc_p, 16);
+        acc_p += __shfl_xor(acc_p, 32);
+        acc_l += __shfl_xor(acc_l, 16);
+        acc_l += __shfl_xor(acc_l, 32);
       }
-      if (lane == 0) out[0] = acc_l;
+      lds_barrier();
+      double* out = a.rootsums + ((size_t)k * a.nchunks + part) * (1 + S + C);
+      if (h == 0 && c == 0) {
+        for (int s = lane; s < S; s += 64) {
+          double tsum = 0.0;
+          for (int cc = 0; cc < C; ++cc) tsum += red[cc * SP + s];
+          out[1 + s] = tsum;
+        }
+        if (lane == 0) out[0] = acc_l;
+      }
+      if (h == 0 && lane == 0) out[1 + S + c] = acc_p;
+      acc_l = acc_p = 0.0;
     }
-    if (h == 0 && lane == 0) out[1 + S + c] = acc_p;
   }
 }
 
@@ -1511,13 +1520,14 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   HX_REQUIRE((size_t)(a.N + 16) * a.C * S + 64 < ((size_t)1 << 31), HX_ERR_UNSUPPORTED,
              "dense-state slab exceeds 31-bit offsets");
   dim3 grid(a.nchunks, a.K, width);
+  PassArgs<R> b = a;
 #define HX_MF(KER, MTV, KVV, TV, RV, ...)                                                    \
   do {                                                                                       \
     auto kern = KER<R, MTV, KVV, TV, RV, SPLIT, ##__VA_ARGS__>;                              \
     if (lds > 64 * 1024)                                                                     \
       HX_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                    \
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
-    kern<<<grid, threads, lds, st>>>(a, nodes, S);                                           \
+    kern<<<grid, threads, lds, st>>>(b, nodes, S);                                           \
   } while (0)
 #define HX_MF_ALL(KER, MTV, KVV, ...)                                                        \
   if (tips == HX_TIPS_CODES) {                                                               \
@@ -1546,7 +1556,6 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
                "dense-state post-order LDS exceeds 64 KiB");
     // (at most 36 KiB)
     const size_t lds_r = lds_b + (sizeof(R) == 4 ? (size_t)a.C * kTile * (16 * MT + 4) * 4 : 0);
-    PassArgs<R> b = a;
     b.tiles_per_chunk = post_level_tiles(a.ntiles, S, a.C, a.K, width, sizeof(R) == 8,
                                          sizeof(R) == 4 && !SPLIT && tips == HX_TIPS_CODES ? 3 : 2);
     grid.x = (a.ntiles + b.tiles_per_chunk - 1) / b.tiles_per_chunk;
@@ -1568,6 +1577,9 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
     }
 #undef HX_MFR
   } else if (post) {
+    const int tb = post_level_tiles(a.ntiles, S, a.C, a.K, width, sizeof(R) == 8);
+    b.root_parts = tb > a.tiles_per_chunk ? tb / a.tiles_per_chunk : 1;
+    grid.x = (a.nchunks + b.root_parts - 1) / b.root_parts;
     if (MT == 1) {
       HX_MF_ROOT(1, 4)
     } else if (MT == 2) {
