@@ -2,6 +2,7 @@
 //   tiles S ntiles C K width f64    -> post_level_tiles
 //   tau ntiles C tiles_per_chunk    -> tau_chunk_tiles
 //   dwalk S C I levels ntiles K     -> use_dwalk
+//   nat S C split post ntiles       -> use_nat_rows
 #include <cstdio>
 #include <cstring>
 
@@ -22,6 +23,10 @@ int main() {
       int S, C, I, h, nt, K;
       if (std::scanf("%d %d %d %d %d %d", &S, &C, &I, &h, &nt, &K) != 6) return 1;
       std::printf("%d\n", (int)hx::use_dwalk(S, C, I, h, nt, K));
+    } else if (!std::strcmp(what, "nat")) {
+      int S, C, f, post, nt;
+      if (std::scanf("%d %d %d %d %d", &S, &C, &f, &post, &nt) != 5) return 1;
+      std::printf("%d\n", (int)hx::use_nat_rows(S, C, f != 0, post != 0, nt));
     } else {
       return 1;
     }

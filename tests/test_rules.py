@@ -70,3 +70,18 @@ def test_post_level_tiles_of_one_category_stay_short(ask, S):
             for w in (1, 9, 64) for f in (0, 1)]
     for q, t in zip(grid, ask(grid)):
         assert 1 <= t <= min(q[2], 10), q
+
+
+def test_rows_as_operands_where_they_are_short_or_used_once(ask):
+    """Past 20 states rows always; one tile's post-order of 20 and fewer never; split products of 17 and
+    19 states never."""
+    for S in range(2, 65):
+        for C in (1, 2, 3, 4):
+            for split in (0, 1):
+                pre, one, many = ask([("nat", S, C, split, 0, 1), ("nat", S, C, split, 1, 1),
+                                      ("nat", S, C, split, 1, 400)])
+                assert pre == many
+                if S > 20:
+                    assert one == many == 1
+                else:
+                    assert one == 0 and not (many and split and S in (17, 19))

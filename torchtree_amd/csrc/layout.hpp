@@ -158,8 +158,13 @@ inline int post_level_tiles(int ntiles, int S, int C, int K, int width, bool f64
 // categories 0.80 to 1.21 and 0.87 to 1.05 (the larger ones at sizes that walk), with 4 0.99 to 1.29
 // and 1.02 to 1.12; 16 states with several categories 0.94 to 1.24 and 0.91 to 1.26; 27 states 0.88
 // to 1.10 and 0.95 to 1.11, 32 0.96 to 1.66 and 0.98 to 1.40.
-inline bool use_nat_rows(int S, int C) {
-  return S > 20 || (S > 16 ? C >= 4 : S > 12 && C >= 2);
+// Split products of 17 and 19 states gain nothing by rows either (4 categories 1.03 to 1.19), and up to
+// 20 states the post-order of a single tile takes operands: its P is used once, and comes faster so
+// (1.04 to 1.33 with rows).
+inline bool use_nat_rows(int S, int C, bool split, bool post, int ntiles) {
+  if (S > 20) return true;
+  if (post && ntiles == 1) return false;
+  return S > 16 ? C >= 4 && !(split && S % 2) : S > 12 && C >= 2;
 }
 
 // Whether a dense FP32 or split-BF16 post-order runs as one walk of the tree (pruning_dwalk.hip) or

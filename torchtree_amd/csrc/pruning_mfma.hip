@@ -613,10 +613,11 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
     if constexpr (kNat) return NR(vslab + c * S, CS, a.N, S, lane);
     else return 0;
   }();
-  if constexpr (kNat) {
-    rows.load(t0, 0, code, nrow);
-    code = code_of(min(t0 + 1, t1 - 1));
-  }
+  // split products, whose forward product is too short to hide them, have operand rows a tile ahead too
+  constexpr bool kOpAhead = !kNat && SPLIT;
+  if constexpr (kNat) rows.load(t0, 0, code, nrow);
+  if constexpr (kOpAhead) post_rows(t0, code, arow);
+  if constexpr (kNat || kOpAhead) code = code_of(min(t0 + 1, t1 - 1));
 
   for (int tile = t0; tile < t1; ++tile) {
     const int nbase = tile * kTile;
@@ -630,17 +631,21 @@ __global__ __launch_bounds__(512) void k_post_mfma_r(PassArgs<R> a,
       code = code_of(min(tile + 2, t1 - 1));
       lds_run<KV>(lt + nn * LS + g * KV, arow);
     } else {
-      post_rows(tile, code, arow);
+      if constexpr (!kOpAhead) post_rows(tile, code, arow);
       const bool rok = nbase + nn < a.N;
 #pragma unroll
       for (int q = 0; q < KV; ++q) arow[q] = (rok && g * KV + q < S) ? arow[q] : R(0);
-      code = code_of(min(tile + 1, t1 - 1));
+      if constexpr (!kOpAhead) code = code_of(min(tile + 1, t1 - 1));
     }
     const float sv = (float)sq[min(nbase + (lane & 15), a.N - 1)] * qmask;
     vec4_t<R> acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = vec4_t<R>{R(0), R(0), R(0), R(0)};
     fp.product(arow, acc);
+    if constexpr (kOpAhead) {  // (the last tile reads its own again, unused)
+      post_rows(min(tile + 1, t1 - 1), code, arow);
+      code = code_of(min(tile + 2, t1 - 1));
+    }
     // lane (nn, g): acc[t][r] = Y[m = acc_row(g, r)][i = 16 t + nn]
     if (h == 1) {
 #pragma unroll
@@ -1505,7 +1510,7 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   const int MT = S <= 16 ? 1 : (S <= 32 ? 2 : 4);
   const int threads = 2 * a.C * 64;
   const size_t lds = mfma_lds<R>(a.C, S, !post);
-  const bool nat = sizeof(R) == 4 && use_nat_rows(S, a.C);
+  const bool nat = sizeof(R) == 4 && use_nat_rows(S, a.C, SPLIT, post, a.ntiles);
   // the kernels stage no codes; a chunk whose codes would not fit beside unpadded tiles is refused as
   // it was when they did
   const size_t codes = 2 * (size_t)a.tiles_per_chunk * kTile;
