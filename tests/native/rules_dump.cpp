@@ -2,6 +2,7 @@
 //   tiles S ntiles C K width f64    -> post_level_tiles
 //   tau ntiles C tiles_per_chunk    -> tau_chunk_tiles
 //   dwalk S C I levels ntiles K     -> use_dwalk
+//   route S C I levels ntiles K dense split -> use_dwalk
 //   nat S C split post ntiles       -> use_nat_rows
 #include <cstdio>
 #include <cstring>
@@ -23,6 +24,10 @@ int main() {
       int S, C, I, h, nt, K;
       if (std::scanf("%d %d %d %d %d %d", &S, &C, &I, &h, &nt, &K) != 6) return 1;
       std::printf("%d\n", (int)hx::use_dwalk(S, C, I, h, nt, K));
+    } else if (!std::strcmp(what, "route")) {
+      int S, C, I, h, nt, K, d, f;
+      if (std::scanf("%d %d %d %d %d %d %d %d", &S, &C, &I, &h, &nt, &K, &d, &f) != 8) return 1;
+      std::printf("%d\n", (int)hx::use_dwalk(S, C, I, h, nt, K, d != 0, f != 0));
     } else if (!std::strcmp(what, "nat")) {
       int S, C, f, post, nt;
       if (std::scanf("%d %d %d %d %d", &S, &C, &f, &post, &nt) != 5) return 1;

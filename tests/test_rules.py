@@ -85,3 +85,11 @@ def test_rows_as_operands_where_they_are_short_or_used_once(ask):
                     assert one == many == 1
                 else:
                     assert one == 0 and not (many and split and S in (17, 19))
+
+
+@pytest.mark.parametrize("S,C", [(8, 4), (17, 2), (18, 1), (18, 2), (19, 4), (24, 3), (32, 2)])
+def test_dense_tips_of_many_patterns_go_by_level(ask, S, C):
+    """Rows of dense tips come word by word in the walk: a large batch on a balanced tree goes by level,
+    which the same call with 20 states does not."""
+    assert ask([("route", S, C, 199, 8, 625, 16, 1, f) for f in (0, 1)]) == [0, 0]
+    assert ask([("route", 20, C, 199, 8, 625, 16, 1, f) for f in (0, 1)]) == [1, 1]

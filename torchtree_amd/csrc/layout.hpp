@@ -173,24 +173,45 @@ inline bool use_nat_rows(int S, int C, bool split, bool post, int ntiles) {
 //   walk   8 + I (a + b C max(0, B - 256)): a node's chain a, whatever there is in flight up to a
 //          block per CU, then the blocks' work. The states decide how P comes (pruning_dwalk.hip):
 //          20 in 16-byte loads, the other sizes word by word, and rows of a multiple of 8 states
-//          (past 20; of 16 with several categories) fall on the same banks.
+//          (past 20; of 16 with several categories) fall on the same banks. So do the rows of dense
+//          tips, which come word by word at every size but 20 and weigh on the chain past 8 states.
 //   levels (launch) x levels + I B C v.
-// Measured at 12 state counts of 2 to 32, 1 to 4 categories, 8 to 350 taxa (caterpillars to balanced
-// trees), 1 to 100000 patterns and 1 to 32 samples, 7870 calls: the slower one costs more than 10 % in
-// 59 of them (at most 42 %); with the walk everywhere 350 taxa x 60 patterns, 27 states, 4 categories
-// took 1068 us (levels 112), 128 x 400 at 20 states 163 (60).
+// Measured at 2 to 32 states, 1 to 4 categories, coded and dense tips, 4 to 500 taxa (caterpillars to
+// balanced trees), 1 to 100000 patterns and 1 to 32 samples, 7820 calls: the slower one costs more than
+// 10 % in 91 of them and 20 % in 28, at most 51 % (4 taxa, where the root is a third of a call); with the walk everywhere 350 taxa x 60 patterns, 27
+// states, 4 categories took 1068 us (levels 112), 128 x 400 at 20 states 163 (60); with coded tips'
+// constants for dense ones 200 x 10000 at 16 samples, 18 states, 2 categories 5674 (3961).
 constexpr int kDwalkMaxS = 32;
-inline bool use_dwalk(int S, int C, int I, int levels, int ntiles, int K) {
+inline bool use_dwalk(int S, int C, int I, int levels, int ntiles, int K, bool dense = false,
+                      bool split = false) {
   if (S > kDwalkMaxS) return false;
   const double blocks = (double)ntiles * K, past = blocks > 256 ? blocks - 256 : 0;
-  double a, b;
-  if (S <= 16) a = 0.73 + 0.08 * C, b = S == 16 && C > 1 ? 0.001 : 0.0005;
-  else if (S < 20) a = 0.8 + 0.27 * C, b = 0.0009;
-  else if (S == 20) a = 0.84 + 0.1 * C, b = 0.0006;
-  else a = 0.95 + 0.47 * C, b = S % 8 == 0 ? 0.003 : 0.0019;
-  const double launch = S <= 16 ? 4.0 + 0.08 * C : (S <= 20 ? 3.95 + 0.37 * C : 4.7 + 0.22 * C);
-  const double v = S <= 16 ? 0.00065 : (S <= 20 ? (C < 4 ? 0.0014 : 0.00115) : 0.0016);
-  return 8 + I * (a + b * C * past) <= levels * launch + I * blocks * C * v;
+  const bool eights = S % 8 == 0;
+  double a, b, launch, v;  // b and v in 1e-4 us
+  if (S <= 16) {
+    a = 0.73 + 0.08 * C, launch = 4.0 + 0.08 * C;
+    b = S == 16 && C > 1 ? 10 : 5, v = 6.5;
+    if (dense) {
+      if (C > 2 && S >= 8) a += (S == 16 ? 0.3 : 0.1) * (C - 2);
+      b = S == 16 ? 17.5 : (S == 8 ? 12.5 : (S > 8 ? 8.5 : 5.5));
+      if (S >= 8) v = 8.8;
+    }
+  } else if (S == 20) {
+    a = 0.84 + 0.1 * C, launch = 3.95 + 0.37 * C;
+    b = 6, v = C < 4 ? 14 : 11.5;
+  } else if (S < 20) {
+    a = 0.8 + 0.27 * C, launch = 3.95 + 0.37 * C;
+    b = dense ? 12 : 11, v = dense ? 11 : (C < 4 ? 13.5 : 12);
+    if (split && !dense) b = 12.8, v = C == 2 || C == 3 ? 12 : 13;
+  } else {
+    a = 0.95 + 0.47 * C, launch = 4.7 + 0.22 * C;
+    b = eights ? 1.24 * S : 17 + 0.7 * (S - 21), v = C == 3 ? 18 : 16;
+    if (dense) {
+      if (C > 2) a += (eights ? 0.75 : 0.3) * (C - 2);
+      b += eights ? 14 : 6, v = C == 3 ? 17 : 14.5;
+    }
+  }
+  return 8 + I * (a + 1e-4 * b * C * past) <= levels * launch + 1e-4 * I * blocks * C * v;
 }
 
 // Tiles per chunk of FP32 d/dtau at 33..64 states. A block's result is C doubles, so its chunk need not

@@ -246,7 +246,8 @@ static bool runs_pre_walk64(const CallArgs& c) {
 // Whether a dense-state call's post-order runs as the walk of pruning_dwalk.hip.
 static bool runs_dwalk(const CallArgs& c) {
   return c.dtype != HX_F64 && use_mfma(c.C, c.S, c.dtype) &&
-         use_dwalk(c.S, c.C, c.plan->I, (int)c.plan->post_off.size() - 1, (c.N + 15) / 16, c.K);
+         use_dwalk(c.S, c.C, c.plan->I, (int)c.plan->post_off.size() - 1, (c.N + 15) / 16, c.K,
+                   c.tip_kind != HX_TIPS_CODES, c.dtype == HX_F32_BF16X3);
 }
 
 template <typename R>
