@@ -151,20 +151,23 @@ inline int post_level_tiles(int ntiles, int S, int C, int K, int width, bool f64
 }
 
 // Whether the FP32 level kernels move rows with lanes along the states (NatRows) or load them as
-// operands, a lane per pattern. Up to 12 states, and up to 20 with few categories, rows are short:
+// operands, a lane per pattern. Below 16 states, and up to 20 with few categories, rows are short:
 // most lanes of a row load idle, and an operand load takes few lines. Operands against rows, the
 // post- and the pre-order of 50 to 350 taxa x 60 to 20000 patterns: 2 and 8 states 0.80 to 1.02 and
 // 0.84 to 1.05 (split products to 1.15, at 3000 patterns x 8 samples), 18 and 20 states with 1 to 3
 // categories 0.80 to 1.21 and 0.87 to 1.05 (the larger ones at sizes that walk), with 4 0.99 to 1.29
-// and 1.02 to 1.12; 16 states with several categories 0.94 to 1.24 and 0.91 to 1.26; 27 states 0.88
-// to 1.10 and 0.95 to 1.11, 32 0.96 to 1.66 and 0.98 to 1.40.
+// and 1.02 to 1.12; 16 states with several categories (50 to 200 taxa x 400 to 20000 patterns) 1.08 to
+// 1.52 and, whole gradients, 1.00 to 1.49, but 13 to 15 states, whose rows straddle lines, 0.91 to 1.06
+// and 0.90 to 1.13, the latter with dense tips and split products alone; 27 states 0.88 to 1.10 and 0.95
+// to 1.11, 32 0.96 to 1.66 and 0.98 to 1.40.
+//
 // Split products of 17 and 19 states gain nothing by rows either (4 categories 1.03 to 1.19), and up to
 // 20 states the post-order of a single tile takes operands: its P is used once, and comes faster so
 // (1.04 to 1.33 with rows).
 inline bool use_nat_rows(int S, int C, bool split, bool post, int ntiles) {
   if (S > 20) return true;
   if (post && ntiles == 1) return false;
-  return S > 16 ? C >= 4 && !(split && S % 2) : S > 12 && C >= 2;
+  return S > 16 ? C >= 4 && !(split && S % 2) : S == 16 && C >= 2;
 }
 
 // Whether a dense FP32 or split-BF16 post-order runs as one walk of the tree (pruning_dwalk.hip) or
