@@ -3,7 +3,7 @@
 //   tau ntiles C tiles_per_chunk    -> tau_chunk_tiles
 //   dwalk S C I levels ntiles K     -> use_dwalk
 //   route S C I levels ntiles K dense split -> use_dwalk
-//   nat S C split post ntiles       -> use_nat_rows
+//   nat S C split post ntiles dense -> use_nat_rows
 #include <cstdio>
 #include <cstring>
 
@@ -29,9 +29,9 @@ int main() {
       if (std::scanf("%d %d %d %d %d %d %d %d", &S, &C, &I, &h, &nt, &K, &d, &f) != 8) return 1;
       std::printf("%d\n", (int)hx::use_dwalk(S, C, I, h, nt, K, d != 0, f != 0));
     } else if (!std::strcmp(what, "nat")) {
-      int S, C, f, post, nt;
-      if (std::scanf("%d %d %d %d %d", &S, &C, &f, &post, &nt) != 5) return 1;
-      std::printf("%d\n", (int)hx::use_nat_rows(S, C, f != 0, post != 0, nt));
+      int S, C, f, post, nt, d;
+      if (std::scanf("%d %d %d %d %d %d", &S, &C, &f, &post, &nt, &d) != 6) return 1;
+      std::printf("%d\n", (int)hx::use_nat_rows(S, C, f != 0, post != 0, nt, d != 0));
     } else {
       return 1;
     }

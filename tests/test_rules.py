@@ -73,14 +73,16 @@ def test_post_level_tiles_of_one_category_stay_short(ask, S):
 
 
 def test_rows_as_operands_where_they_are_short_or_used_once(ask):
-    """Past 20 states rows always; one tile's post-order of 20 and fewer never; below 16 states and with
+    """Past 20 states rows, but with coded tips at 3 categories; one tile's post-order of 20 and fewer never; below 16 states and with
     split products of 17 and 19 never."""
     for S in range(2, 65):
         for C in (1, 2, 3, 4):
             for split in (0, 1):
-                pre, one, many = ask([("nat", S, C, split, 0, 1), ("nat", S, C, split, 1, 1),
-                                      ("nat", S, C, split, 1, 400)])
+                pre, one, many = ask([("nat", S, C, split, 0, 1, 1), ("nat", S, C, split, 1, 1, 1),
+                                      ("nat", S, C, split, 1, 400, 1)])
                 assert pre == many
+                coded = ask([("nat", S, C, split, 0, 1, 0), ("nat", S, C, split, 1, 400, 0)])
+                assert coded == [pre, many and not (20 < S < 32 and C == 3 and not split)]
                 if S > 20:
                     assert one == many == 1
                 else:

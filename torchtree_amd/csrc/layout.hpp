@@ -163,9 +163,11 @@ inline int post_level_tiles(int ntiles, int S, int C, int K, int width, bool f64
 //
 // Split products of 17 and 19 states gain nothing by rows either (4 categories 1.03 to 1.19), and up to
 // 20 states the post-order of a single tile takes operands: its P is used once, and comes faster so
-// (1.04 to 1.33 with rows).
-inline bool use_nat_rows(int S, int C, bool split, bool post, int ntiles) {
-  if (S > 20) return true;
+// (1.04 to 1.33 with rows). With coded tips, whose rows come from the table's few lines either way, the
+// post-order of 21 to 31 states does too at one tile (0.97 to 1.18 with rows) and with FP32 products at 3
+// categories, whose blocks of 6 waves leave the rows' latency bare (1.00 to 1.16).
+inline bool use_nat_rows(int S, int C, bool split, bool post, int ntiles, bool dense) {
+  if (S > 20) return !(post && !dense && S < 32 && (ntiles == 1 || (C == 3 && !split)));
   if (post && ntiles == 1) return false;
   return S > 16 ? C >= 4 && !(split && S % 2) : S == 16 && C >= 2;
 }

@@ -1510,7 +1510,7 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
   const int MT = S <= 16 ? 1 : (S <= 32 ? 2 : 4);
   const int threads = 2 * a.C * 64;
   const size_t lds = mfma_lds<R>(a.C, S, !post);
-  const bool nat = sizeof(R) == 4 && use_nat_rows(S, a.C, SPLIT, post, a.ntiles);
+  const bool nat = sizeof(R) == 4 && use_nat_rows(S, a.C, SPLIT, post, a.ntiles, tips != HX_TIPS_CODES);
   // the kernels stage no codes; a chunk whose codes would not fit beside unpadded tiles is refused as
   // it was when they did
   const size_t codes = 2 * (size_t)a.tiles_per_chunk * kTile;
@@ -1578,7 +1578,7 @@ static int launch_mfma_t(bool post, const PassArgs<R>& a, const int32_t* nodes, 
     } else if (S <= 20) {
       HX_MF_NAT(HX_MFR, 2, 5)
     } else {
-      HX_MFR(2, 8, sizeof(R) == 4)
+      HX_MF_NAT(HX_MFR, 2, 8)
     }
 #undef HX_MFR
   } else if (post) {
