@@ -132,10 +132,25 @@ inline Tiling make_tiling(int N, int C, int K, int S, int rb) {
 // them at most and mostly ahead; rounds of one block per CU were 0 to 73 % behind. FP64, 2 states, 4
 // categories, 50 taxa x 3000 patterns at 8 samples: 570 us in such rounds, 348 in the gradient's
 // chunks, 333 now; 20 states, 128 x 20000: 1773 in such rounds, 1556 now.
+//
+// FP64 past 16 states holds 5 or 4 waves on a SIMD, so that a level of a few thousand blocks takes a few
+// rounds of the chip, and a nearly empty last one shows: with up to four, t is the one with the least
+// rounds (t + 1). 25 to 60 taxa, caterpillars, 4000 to 20000 patterns, 4 and 8 samples, 20 to 32 states, 2 to 4
+// categories: 0.73 to 0.87 of the time without.
 inline int post_level_tiles(int ntiles, int S, int C, int K, int width, bool f64, int waves = 2) {
   if (S <= 32) {
-    const double q = S <= 16 ? 4096.0 : (S <= 20 && C <= 2 ? 2048.0 : 1024.0);
-    const double t = sqrt((double)ntiles * K * width * C / q);
+    const double q = S <= 16 ? 4096.0 : (S <= 20 ? 2048.0 : 1024.0);
+    double t = sqrt((double)ntiles * K * width * C / q);
+    if (f64 && S > 16 && C > 1) {
+      const int simd = S <= 20 ? 5 : 4;  // waves of the kernel on a SIMD
+      const double slots = 256.0 * (C == 2 ? simd : simd / 2);
+      auto blocks = [&](double u) { return ceil(ntiles / u) * K * width; };
+      auto cost = [&](double u) { return ceil(blocks(u) / slots) * (u + 1.0); };
+      if (t < 1.0) t = 1.0;
+      if (blocks(t) <= 4.0 * slots)
+        for (int u = 1; u <= ntiles && u <= 64; ++u)
+          if (cost(u) < cost(t)) t = u;
+    }
     const int nch = (int)(ntiles / (t < 1.0 ? 1.0 : t) + 0.5), least = (ntiles + 63) / 64;
     return (ntiles + (nch > least ? nch : least) - 1) / (nch > least ? nch : least);  // even chunks
   }
